@@ -14,6 +14,7 @@
 // allocation of this library or of torch is.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <string>
@@ -186,20 +187,52 @@ int matmul_check(kraken_hip_context* ctx, int format, const kraken_buffer& weigh
   return KRAKEN_OK;
 }
 
+// Whether a product of more than 8 tokens runs as kquant_mm.hip's two launches:
+// the faster form for `rows` (the largest matrix of a group), no form forced
+// through KRAKEN_KQUANT_GEMM, and a workspace that holds its packed inputs or
+// can grow to (not while the stream is captured, where an allocation would end
+// the capture; the other forms of a Q4_K product need no workspace).
+bool takes_mm(kraken_hip_context* ctx, int format, size_t rows, size_t cols, size_t tokens) {
+  if (!kquant_mm_supported(format, rows, cols, tokens) ||
+      std::getenv("KRAKEN_KQUANT_GEMM") != nullptr) {
+    return false;
+  }
+  if (ctx->validation_only || kquant_mm_workspace_bytes(cols, tokens) <= ctx->workspace_bytes) {
+    return true;
+  }
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(ctx->stream, &capture) == hipSuccess &&
+         capture == hipStreamCaptureStatusNone;
+}
+
+// launch_kquant_mm or launch_kquant_matmul for one matrix, with the workspace.
+int run_matmul(kraken_hip_context* ctx, int format, const std::string& p, const void* weight,
+               size_t rows, size_t cols, size_t tokens, const float* input, const float* up,
+               const float* residual, float* output) {
+  const bool mm = takes_mm(ctx, format, rows, cols, tokens);
+  KRAKEN_TRY(ensure_workspace(
+    ctx, mm ? kquant_mm_workspace_bytes(cols, tokens)
+            : kquant_matmul_workspace_bytes(format, rows, cols, tokens, up != nullptr)));
+  KRAKEN_TRY(begin_launch(ctx));
+  const hipError_t e =
+    mm ? launch_kquant_mm(format, 1, &weight, &rows, cols, tokens, input, up, residual, &output,
+                          ctx->workspace, ctx->workspace_bytes, ctx->stream)
+       : launch_kquant_matmul(format, weight, rows, cols, tokens, input, output, ctx->workspace,
+                              ctx->workspace_bytes, ctx->stream, up, residual);
+  if (e != hipSuccess) {
+    return internal(p + "launch failed: " + hipGetErrorString(e));
+  }
+  return finish_launch(ctx, (p + "command failed: ").c_str());
+}
+
 int matmul_entry(kraken_hip_context* ctx, int format, const kraken_buffer& weight, size_t rows,
                  size_t cols, size_t tokens, const kraken_buffer& input,
                  const kraken_buffer& output) {
   KRAKEN_TRY(matmul_check(ctx, format, weight, rows, cols, tokens, input, output));
   const std::string p = std::string("HIP ") + fmt_name(format) + " matmul ";
-  KRAKEN_TRY(ensure_workspace(ctx, kquant_matmul_workspace_bytes(format, rows, cols, tokens)));
-  KRAKEN_TRY(begin_launch(ctx));
-  const hipError_t e = launch_kquant_matmul(
-    format, weight.data, rows, cols, tokens, static_cast<const float*>(input.data),
-    static_cast<float*>(output.data), ctx->workspace, ctx->workspace_bytes, ctx->stream);
-  if (e != hipSuccess) {
-    return internal(p + "launch failed: " + hipGetErrorString(e));
-  }
-  return finish_launch(ctx, (p + "command failed: ").c_str());
+  return run_matmul(ctx, format, p, weight.data, rows, cols, tokens,
+                    static_cast<const float*>(input.data), nullptr, nullptr,
+                    static_cast<float*>(output.data));
 }
 
 // dequantize_row_q*_k_f32 (mps_backend.mm:7217-7283).
@@ -569,17 +602,9 @@ KRAKEN_API int kraken_hip_kquant_matmul_fused_f32(kraken_hip_context* ctx, uint3
     }
   }
   const std::string p = std::string("HIP ") + fmt_name(format) + " fused matmul ";
-  KRAKEN_TRY(ensure_workspace(
-    ctx, kquant_matmul_workspace_bytes(format, rows, cols, tokens, up.data != nullptr)));
-  KRAKEN_TRY(begin_launch(ctx));
-  const hipError_t e = launch_kquant_matmul(
-    format, weight.data, rows, cols, tokens, static_cast<const float*>(input.data),
-    static_cast<float*>(output.data), ctx->workspace, ctx->workspace_bytes, ctx->stream,
-    static_cast<const float*>(up.data), static_cast<const float*>(residual.data));
-  if (e != hipSuccess) {
-    return internal(p + "launch failed: " + hipGetErrorString(e));
-  }
-  return finish_launch(ctx, (p + "command failed: ").c_str());
+  return run_matmul(ctx, format, p, weight.data, rows, cols, tokens,
+                    static_cast<const float*>(input.data), static_cast<const float*>(up.data),
+                    static_cast<const float*>(residual.data), static_cast<float*>(output.data));
 }
 
 KRAKEN_API int kraken_hip_kquant_matmul_multi_f32(kraken_hip_context* ctx, size_t count,
@@ -611,10 +636,17 @@ KRAKEN_API int kraken_hip_kquant_matmul_multi_f32(kraken_hip_context* ctx, size_
   }
   const char* group = std::getenv("KRAKEN_KQUANT_GROUP");
   if (same_format && (group == nullptr || std::strcmp(group, "off") != 0)) {
+    const bool mm = takes_mm(ctx, formats[0], *std::max_element(rows, rows + count), cols, tokens);
+    if (mm) {
+      KRAKEN_TRY(ensure_workspace(ctx, kquant_mm_workspace_bytes(cols, tokens)));
+    }
     KRAKEN_TRY(begin_launch(ctx));
+    const float* x = static_cast<const float*>(input.data);
     const hipError_t e =
-      launch_kquant_matmul_group(formats[0], count, w, rows, cols, tokens,
-                                 static_cast<const float*>(input.data), out, ctx->stream);
+      mm ? launch_kquant_mm(formats[0], count, w, rows, cols, tokens, x, nullptr, nullptr, out,
+                            ctx->workspace, ctx->workspace_bytes, ctx->stream)
+         : launch_kquant_matmul_group(formats[0], count, w, rows, cols, tokens, x, out,
+                                      ctx->stream);
     if (e == hipSuccess) {
       return finish_launch(ctx, "HIP K-quant multi matmul command failed: ");
     }

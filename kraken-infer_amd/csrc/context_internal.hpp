@@ -327,6 +327,17 @@ hipError_t launch_kquant_matmul(int format, const void* weight, size_t rows, siz
                                 size_t tokens, const float* input, float* output,
                                 void* workspace, size_t workspace_bytes, hipStream_t stream,
                                 const float* up = nullptr, const float* residual = nullptr);
+// The two launches of kquant_mm.hip (input packing, then the product with the
+// weights decoded in registers): up to kKquantGroupMax matrices of one format
+// over the same input, with `up` as above; `residual` with one matrix only.
+// supported: whether this is the faster form for that many rows (of the group's
+// largest matrix).
+bool kquant_mm_supported(int format, size_t rows, size_t cols, size_t tokens);
+size_t kquant_mm_workspace_bytes(size_t cols, size_t tokens);
+hipError_t launch_kquant_mm(int format, size_t count, const void* const* weights,
+                            const size_t* rows, size_t cols, size_t tokens, const float* input,
+                            const float* up, const float* residual, float* const* outputs,
+                            void* workspace, size_t workspace_bytes, hipStream_t stream);
 // Up to kKquantGroupMax matmuls of one format that share input, cols and
 // tokens (kquant.hip).  More than kKquantGemvMaxTokens tokens with the fused
 // GEMM form (weights decoded in the B tile) run as one launch whose grid holds
