@@ -1016,12 +1016,55 @@ struct SplitPlan {
 constexpr uint64_t kRaggedKeysPerSplit = 1024;
 constexpr uint64_t kSingleSplitKeys = 256;
 
+bool aligned16(const void* ptr) { return ((uintptr_t)ptr & 15u) == 0; }
+
+// The tuned kernel moves 16-byte chunks; shapes or pointers outside that contract
+// take the generic kernel.
+bool tuned_args(const AttentionArgs& a) {
+  const uint32_t d = a.head_dim;
+  const uint32_t g = a.heads / a.kv_heads;
+  if (!aligned16(a.query) || !aligned16(a.key_cache) || !aligned16(a.value_cache) ||
+      !aligned16(a.output)) {
+    return false;
+  }
+  return (d == 256 || d == 128 || d == 64) && (g == 1 || g == 2 || g == 4 || g == 8);
+}
+
+// Whether the several-token kernel runs: a sequence's 2 or more tokens with
+// head_dim 256, an f16 cache and up to 4 query heads per KV head, where one
+// workgroup per token would read many K/V rows again.  Its own launch takes about
+// 2 us longer on a short context, so the line lies at the rows that the tokens
+// read together.  Measured, us per call with prologue and merge, one workgroup per
+// token / this kernel (2 KV heads x 4; 4 x 2 query heads):
+//   37 tokens after  1500: 29.0 / 19.5;  41.0 / 19.5
+//   16 tokens after  1500: 16.8 / 18.5;  20.2 / 18.4   (48k and 97k rows)
+//   63 tokens after   200: 16.8 / 16.2;  15.9 / 16.3   (33k and 66k rows)
+//    3 tokens after  6144: 17.4 / 15.9;  21.5 / 15.9   (37k and 74k rows)
+//    2 tokens after  6144: 14.7 / 14.9;  16.9 / 15.1   (25k and 49k rows)
+//   37 tokens after  6144: 59.3 / 25.0; 122.7 / 25.9
+//   63 tokens after 16384:  174 / 46.6;   295 / 46.3
+// KRAKEN_DECODE_KERNEL forces one of the other kernels.
+bool takes_rows(const AttentionArgs& a) {
+  const uint32_t g = a.heads / a.kv_heads;
+  const uint64_t keys = (uint64_t)a.start_position + a.tokens;
+  const uint64_t rows = keys * a.tokens * a.kv_heads;
+  return a.seq_positions == nullptr && a.tokens >= 2 && a.head_dim == (uint32_t)kMD && a.kv_f16 &&
+         (g == 1 || g == 2 || g == 4) && tuned_args(a) &&
+         (rows >= 81920u || (keys >= 4096u && rows >= 32768u)) &&
+         std::getenv("KRAKEN_DECODE_KERNEL") == nullptr;
+}
+
 SplitPlan plan_splits(const AttentionArgs& a, int cu_count) {
   const bool ragged = a.seq_positions != nullptr;
   // Keys of the longest query.
   const uint64_t max_keys =
     ragged ? (uint64_t)a.max_position + 1 : (uint64_t)a.start_position + a.tokens;
-  const uint64_t units = (uint64_t)a.tokens * a.kv_heads;
+  // Query rows of a workgroup: one token's heads, or 16 of any.
+  const bool rows = takes_rows(a);
+  const uint64_t group = a.heads / a.kv_heads;
+  const uint64_t units =
+    (rows ? (a.tokens * group + kRowsPerGroup - 1) / kRowsPerGroup : (uint64_t)a.tokens) *
+    a.kv_heads;
   const uint64_t slots = (uint64_t)(cu_count > 0 ? cu_count : 256);
   uint64_t splits_target = slots / units;
   if (splits_target < 1) {
@@ -1039,26 +1082,22 @@ SplitPlan plan_splits(const AttentionArgs& a, int cu_count) {
       kps = (uint64_t)v;
     }
   }
+  if (rows) {
+    // The partials stay within the array that the allocation-free entry has, or
+    // within a smaller limit of the caller's.
+    const uint64_t limit = a.partial_limit < kNoAllocScratchBytes ? a.partial_limit
+                                                                  : kNoAllocScratchBytes;
+    const uint64_t per_split =
+      (uint64_t)a.tokens * a.heads * (a.head_dim + 2u) * sizeof(float);
+    const uint64_t most = std::max<uint64_t>(1, limit / per_split);
+    kps = std::max(kps, most > 1 ? (max_keys + most - 1) / most : max_keys);
+  }
   uint64_t splits = (max_keys + kps - 1) / kps;
   if (splits > kMaxSplits) {
     kps = (max_keys + kMaxSplits - 1) / kMaxSplits;
     splits = (max_keys + kps - 1) / kps;
   }
   return SplitPlan{(uint32_t)kps, (uint32_t)splits};
-}
-
-bool aligned16(const void* ptr) { return ((uintptr_t)ptr & 15u) == 0; }
-
-// The tuned kernel moves 16-byte chunks; shapes or pointers outside that contract
-// take the generic kernel.
-bool tuned_args(const AttentionArgs& a) {
-  const uint32_t d = a.head_dim;
-  const uint32_t g = a.heads / a.kv_heads;
-  if (!aligned16(a.query) || !aligned16(a.key_cache) || !aligned16(a.value_cache) ||
-      !aligned16(a.output)) {
-    return false;
-  }
-  return (d == 256 || d == 128 || d == 64) && (g == 1 || g == 2 || g == 4 || g == 8);
 }
 
 size_t partial_bytes(const AttentionArgs& a, const SplitPlan& plan) {
@@ -1107,26 +1146,8 @@ DecodeKernel decode_kernel_choice(uint32_t keys_per_split, bool ragged) {
   return ragged ? DecodeKernel::vector : DecodeKernel::short_split;
 }
 
-template <int D, int G, typename KV>
-hipError_t launch_tuned(const DecodeParams& p, hipStream_t stream) {
-  // Ragged: one workgroup per work-list entry (see ragged_plan_kernel).
-  const dim3 grid = p.work_items != nullptr ? dim3(p.splits * p.kv_heads * p.tokens)
-                                            : dim3(p.splits, p.kv_heads, p.tokens);
-  DecodeKernel kind = DecodeKernel::vector;
-  if constexpr (D == kMD && std::is_same_v<KV, half_t> && (G == 1 || G == 2 || G == 4)) {
-    kind = decode_kernel_choice(p.keys_per_split, p.work_items != nullptr);
-    if (kind == DecodeKernel::mfma) {
-      attention_decode_mfma_kernel<G><<<grid, 64 * kMWaves, 0, stream>>>(p);
-    } else if (kind == DecodeKernel::short_split) {
-      const hipError_t es = launch_decode_short(p, G, grid, stream);
-      if (es != hipSuccess) {
-        return es;
-      }
-    }
-  }
-  if (kind == DecodeKernel::vector) {
-    attention_decode_kernel<D, G, KV><<<grid, 64 * RowShape<D, KV>::W, 0, stream>>>(p);
-  }
+// The split merge after a decode kernel (none for one split).
+hipError_t combine(const DecodeParams& p, uint32_t head_dim, hipStream_t stream) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || p.splits == 1) {
     return e;
@@ -1140,11 +1161,38 @@ hipError_t launch_tuned(const DecodeParams& p, hipStream_t stream) {
   c.heads = p.heads;
   c.kv_heads = p.kv_heads;
   c.splits = p.splits;
-  c.head_dim = D;
+  c.head_dim = head_dim;
   c.positions = p.seq_positions;
   c.start_position = p.start_position;
   c.keys_per_split = p.keys_per_split;
   return launch_attention_combine(c, stream);
+}
+
+template <int D, int G, typename KV>
+hipError_t launch_tuned(const DecodeParams& p, hipStream_t stream) {
+  // Ragged: one workgroup per work-list entry (see ragged_plan_kernel).
+  const dim3 grid = p.work_items != nullptr ? dim3(p.splits * p.kv_heads * p.tokens)
+                                            : dim3(p.splits, p.kv_heads, p.tokens);
+  DecodeKernel kind = DecodeKernel::vector;
+  if constexpr (D == kMD && std::is_same_v<KV, half_t> && (G == 1 || G == 2 || G == 4)) {
+    if (p.rows) {
+      const hipError_t er = launch_decode_rows(p, G, stream);
+      return er != hipSuccess ? er : combine(p, D, stream);
+    }
+    kind = decode_kernel_choice(p.keys_per_split, p.work_items != nullptr);
+    if (kind == DecodeKernel::mfma) {
+      attention_decode_mfma_kernel<G><<<grid, 64 * kMWaves, 0, stream>>>(p);
+    } else if (kind == DecodeKernel::short_split) {
+      const hipError_t es = launch_decode_short(p, G, grid, stream);
+      if (es != hipSuccess) {
+        return es;
+      }
+    }
+  }
+  if (kind == DecodeKernel::vector) {
+    attention_decode_kernel<D, G, KV><<<grid, 64 * RowShape<D, KV>::W, 0, stream>>>(p);
+  }
+  return combine(p, D, stream);
 }
 
 template <typename KV>
@@ -1484,6 +1532,7 @@ hipError_t launch_attention_decode(const AttentionArgs& a, int cu_count, void* w
     return hipErrorInvalidValue;  // ragged decode runs on the tuned kernel only
   }
   p.splits = 1;
+  p.rows = tuned && takes_rows(a);
   if (tuned) {
     p.keys_per_split = plan.keys_per_split;
     p.splits = plan.splits;

@@ -24,6 +24,7 @@ struct DecodeParams {
   float* part_ml;  // [tokens][kv_heads][splits][G][2]
   uint32_t layer, start_position, tokens, capacity_tokens, heads, kv_heads;
   uint32_t keys_per_split, splits;
+  bool rows;  // the several-token kernel (attention_rows.hip)
   float scale_log2;
   // Ragged multi-sequence mode (see AttentionArgs): per-token K/V element
   // offsets and positions, and the pools' element count.
@@ -109,6 +110,11 @@ hipError_t launch_decode_short(const DecodeParams& p, uint32_t group, dim3 grid,
 // (1, kv_heads, 1).
 hipError_t launch_decode_short_prologue(const DecodeParams& p, const PrologueFold& f,
                                         uint32_t group, hipStream_t stream);
+
+// Launches the several-token kernel (attention_rows.hip) for head_dim 256, an f16
+// cache and G in {1, 2, 4}: kRowsPerGroup query rows per workgroup.
+constexpr uint32_t kRowsPerGroup = 16;
+hipError_t launch_decode_rows(const DecodeParams& p, uint32_t group, hipStream_t stream);
 
 }  // namespace decode
 }  // namespace kraken

@@ -197,12 +197,7 @@ bool takes_mm(kraken_hip_context* ctx, int format, size_t rows, size_t cols, siz
       std::getenv("KRAKEN_KQUANT_GEMM") != nullptr) {
     return false;
   }
-  if (ctx->validation_only || kquant_mm_workspace_bytes(cols, tokens) <= ctx->workspace_bytes) {
-    return true;
-  }
-  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(ctx->stream, &capture) == hipSuccess &&
-         capture == hipStreamCaptureStatusNone;
+  return kquant_mm_workspace_bytes(cols, tokens) <= ctx->workspace_bytes || workspace_can_grow(ctx);
 }
 
 // launch_kquant_mm or launch_kquant_matmul for one matrix, with the workspace.

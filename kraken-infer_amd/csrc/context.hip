@@ -107,6 +107,13 @@ int ensure_workspace(kraken_hip_context* ctx, size_t bytes) {
   return KRAKEN_OK;
 }
 
+bool workspace_can_grow(const kraken_hip_context* ctx) {
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  return ctx->validation_only ||
+         (hipStreamIsCapturing(ctx->stream, &capture) == hipSuccess &&
+          capture == hipStreamCaptureStatusNone);
+}
+
 int check_u32(size_t value, const char* name) {
   if (!fits_u32(value)) {
     return invalid(std::string("HIP ") + name + " exceeds uint32 range");
