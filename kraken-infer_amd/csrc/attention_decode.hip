@@ -1035,14 +1035,15 @@ bool tuned_args(const AttentionArgs& a) {
 // workgroup per token would read many K/V rows again.  Its own launch takes about
 // 2 us longer on a short context, so the line lies at the rows that the tokens
 // read together.  Measured, us per call with prologue and merge, one workgroup per
-// token / this kernel (2 KV heads x 4; 4 x 2 query heads):
-//   37 tokens after  1500: 29.0 / 19.5;  41.0 / 19.5
-//   16 tokens after  1500: 16.8 / 18.5;  20.2 / 18.4   (48k and 97k rows)
-//   63 tokens after   200: 16.8 / 16.2;  15.9 / 16.3   (33k and 66k rows)
-//    3 tokens after  6144: 17.4 / 15.9;  21.5 / 15.9   (37k and 74k rows)
-//    2 tokens after  6144: 14.7 / 14.9;  16.9 / 15.1   (25k and 49k rows)
-//   37 tokens after  6144: 59.3 / 25.0; 122.7 / 25.9
-//   63 tokens after 16384:  174 / 46.6;   295 / 46.3
+// token / this kernel, 2 KV heads x 4 query heads:
+//   37 tokens after  1500: 27.5 / 19.6  (114k rows read together)
+//   16 tokens after  1500: 16.6 / 18.5  ( 49k)
+//   63 tokens after   200: 16.8 / 16.2  ( 33k)
+//    3 tokens after  6144: 17.4 / 16.7  ( 37k)
+//    2 tokens after  6144: 14.5 / 14.9  ( 25k)
+//   37 tokens after  6144: 59.7 / 25.8
+//   63 tokens after 16384:  175 / 50.3
+// (4 x 2: 16 tokens after 1500 20.2 / 18.4, 37 after 6144 123 / 25.9.)
 // KRAKEN_DECODE_KERNEL forces one of the other kernels.
 bool takes_rows(const AttentionArgs& a) {
   const uint32_t g = a.heads / a.kv_heads;

@@ -18,7 +18,8 @@
 // A tile is 48 MFMAs and about 270 other instructions; what bounded the first
 // form was the wait for each of its 24 LDS reads in turn (1.6 us a tile).  All of
 // a tile's K fragments are requested before the first is used, and all of its V
-// fragments before the softmax.
+// fragments before the softmax: 37 tokens after 6144 keys (8 / 2 heads, with
+// prologue and merge) 33.4 -> 25.8 us, from 59.7 with one workgroup per token.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
