@@ -97,20 +97,24 @@ __device__ __forceinline__ void norm_rope(const float v_in[4], const float w[4],
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const uint32_t e = lane + 64u * i;
-    const uint32_t p = e < half_dims ? e + half_dims : (e < n_dims ? e - half_dims : e);
-    const int src_lane = (int)(p & 63u);
-    const uint32_t src_reg = p >> 6;
-    float partner = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float x = __shfl(v[j], src_lane, 64);
-      partner = src_reg == (uint32_t)j ? x : partner;
-    }
     r[i] = v[i];
-    if (e < n_dims) {
-      const double x0 = e < half_dims ? v[i] : partner;
-      const double x1 = e < half_dims ? partner : v[i];
-      r[i] = e < half_dims ? (float)(x0 * cs[i] - x1 * sn[i]) : (float)(x1 * cs[i] + x0 * sn[i]);
+    if (64u * i < n_dims) {  // wave-uniform: the rotation reaches these elements
+      const uint32_t p = e < half_dims ? e + half_dims : (e < n_dims ? e - half_dims : e);
+      const int src_lane = (int)(p & 63u);
+      const uint32_t src_reg = p >> 6;
+      float partner = 0.0f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (64u * j < n_dims) {  // partners lie below n_dims
+          const float x = __shfl(v[j], src_lane, 64);
+          partner = src_reg == (uint32_t)j ? x : partner;
+        }
+      }
+      if (e < n_dims) {
+        const double x0 = e < half_dims ? v[i] : partner;
+        const double x1 = e < half_dims ? partner : v[i];
+        r[i] = e < half_dims ? (float)(x0 * cs[i] - x1 * sn[i]) : (float)(x1 * cs[i] + x0 * sn[i]);
+      }
     }
     // The f32 result kept as such: a caller that rounds it to fp16 (the K
     // append) must not get the norm's last multiply and that rounding fused
