@@ -1044,15 +1044,29 @@ bool tuned_args(const AttentionArgs& a) {
 //   37 tokens after  6144: 59.7 / 25.8
 //   63 tokens after 16384:  175 / 50.3
 // (4 x 2: 16 tokens after 1500 20.2 / 18.4, 37 after 6144 123 / 25.9.)
+// Over an f32 cache, head_dim 64 or 128, the line lies at the multiplications that
+// the tokens' own workgroups do (8 KV heads x 2, head_dim 128):
+//   512 tokens after    0: 73.7 / 21.9;  after 2048: 456 / 99.4
+//   100 tokens after    0:  9.0 /  9.3  (21M);  after 100: 14.2 / 12.8  (41M)
+//    16 tokens after  500: 10.6 / 11.7  (17M)
+//     8 tokens after 2048: 14.6 / 11.9  (34M)
+// (head_dim 64, 4 x 1: 64 tokens after 512 5.9 / 10.0 (9M), 256 after 512 16.6 /
+// 9.5.  At head_dim 256 the operands of two tiles and O do not fit the registers:
+// 512 tokens, 2 x 4 heads 79 / 156.)
 // KRAKEN_DECODE_KERNEL forces one of the other kernels.
 bool takes_rows(const AttentionArgs& a) {
+  if (a.seq_positions != nullptr || a.tokens < 2 || !tuned_args(a) ||
+      std::getenv("KRAKEN_DECODE_KERNEL") != nullptr) {
+    return false;
+  }
   const uint32_t g = a.heads / a.kv_heads;
   const uint64_t keys = (uint64_t)a.start_position + a.tokens;
   const uint64_t rows = keys * a.tokens * a.kv_heads;
-  return a.seq_positions == nullptr && a.tokens >= 2 && a.head_dim == (uint32_t)kMD && a.kv_f16 &&
-         (g == 1 || g == 2 || g == 4) && tuned_args(a) &&
-         (rows >= 81920u || (keys >= 4096u && rows >= 32768u)) &&
-         std::getenv("KRAKEN_DECODE_KERNEL") == nullptr;
+  if (!a.kv_f16) {
+    return a.head_dim < 256u && rows * a.head_dim * g >= (24ull << 20);
+  }
+  return a.head_dim == (uint32_t)kMD && g != 8 &&
+         (rows >= 81920u || (keys >= 4096u && rows >= 32768u));
 }
 
 SplitPlan plan_splits(const AttentionArgs& a, int cu_count) {
@@ -1188,6 +1202,12 @@ hipError_t launch_tuned(const DecodeParams& p, hipStream_t stream) {
       if (es != hipSuccess) {
         return es;
       }
+    }
+  }
+  if constexpr (std::is_same_v<KV, float> && D < 256) {
+    if (p.rows) {
+      const hipError_t er = launch_decode_rows_f32(p, D, G, stream);
+      return er != hipSuccess ? er : combine(p, D, stream);
     }
   }
   if (kind == DecodeKernel::vector) {

@@ -24,7 +24,7 @@ struct DecodeParams {
   float* part_ml;  // [tokens][kv_heads][splits][G][2]
   uint32_t layer, start_position, tokens, capacity_tokens, heads, kv_heads;
   uint32_t keys_per_split, splits;
-  bool rows;  // the several-token kernel (attention_rows.hip)
+  bool rows;  // a several-token kernel (attention_rows.hip, attention_rows_f32.hip)
   float scale_log2;
   // Ragged multi-sequence mode (see AttentionArgs): per-token K/V element
   // offsets and positions, and the pools' element count.
@@ -115,6 +115,10 @@ hipError_t launch_decode_short_prologue(const DecodeParams& p, const PrologueFol
 // cache and G in {1, 2, 4}: kRowsPerGroup query rows per workgroup.
 constexpr uint32_t kRowsPerGroup = 16;
 hipError_t launch_decode_rows(const DecodeParams& p, uint32_t group, hipStream_t stream);
+// The same over an f32 cache (attention_rows_f32.hip), head_dim 64 or 128 and G in
+// {1, 2, 4, 8}.
+hipError_t launch_decode_rows_f32(const DecodeParams& p, uint32_t head_dim, uint32_t group,
+                                  hipStream_t stream);
 
 }  // namespace decode
 }  // namespace kraken
