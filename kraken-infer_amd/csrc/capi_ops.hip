@@ -40,57 +40,44 @@ int attention_entry(kraken_hip_context* ctx, const char* what, bool kv_f16,
                     size_t kv_heads, size_t head_dim, const kraken_buffer& output,
                     bool no_alloc = false, bool query_f16 = false) {
   KRAKEN_TRY(check_context(ctx));
-  const std::string w = std::string("HIP ") + what;
+  const auto w = [what] { return std::string("HIP ") + what; };
   if (tokens == 0 || heads == 0 || kv_heads == 0 || head_dim == 0 || capacity_tokens == 0) {
-    return invalid(w + " dimensions must be positive");
+    return invalid(w() + " dimensions must be positive");
   }
   if (heads % kv_heads != 0) {
-    return invalid(w + " heads must be divisible by kv_heads");
+    return invalid(w() + " heads must be divisible by kv_heads");
   }
   if (head_dim > 256u) {
-    return invalid(w + " head_dim exceeds 256");
+    return invalid(w() + " head_dim exceeds 256");
   }
   size_t key_count = 0;
   if (!checked_add(start_position, tokens, key_count) || key_count > capacity_tokens) {
-    return invalid(w + " chunk exceeds KV cache capacity");
+    return invalid(w() + " chunk exceeds KV cache capacity");
   }
   size_t attn_dim = 0, kv_dim = 0, query_values = 0, cache_layers = 0, cache_values = 0;
   if (!checked_mul(heads, head_dim, attn_dim) || !checked_mul(kv_heads, head_dim, kv_dim) ||
       !checked_mul(tokens, attn_dim, query_values) || layer == SIZE_MAX ||
       !checked_mul(layer + 1u, capacity_tokens, cache_layers) ||
       !checked_mul(cache_layers, kv_dim, cache_values)) {
-    return invalid(w + " value count overflow");
+    return invalid(w() + " value count overflow");
   }
-  const std::string nq = std::string(what) + " query";
-  const std::string nk = std::string(what) + " key cache";
-  const std::string nv = std::string(what) + " value cache";
-  const std::string ng = std::string(what) + " gate";
-  const std::string no = std::string(what) + " output";
   KRAKEN_TRY(validate_buffer(query, query_values, query_f16 ? sizeof(uint16_t) : sizeof(float),
-                             nq.c_str()));
+                             what, " query"));
   const size_t elem = kv_f16 ? sizeof(uint16_t) : sizeof(float);
-  KRAKEN_TRY(validate_buffer(key_cache, cache_values, elem, nk.c_str()));
-  KRAKEN_TRY(validate_buffer(value_cache, cache_values, elem, nv.c_str()));
+  KRAKEN_TRY(validate_buffer(key_cache, cache_values, elem, what, " key cache"));
+  KRAKEN_TRY(validate_buffer(value_cache, cache_values, elem, what, " value cache"));
   if (gate != nullptr) {
-    KRAKEN_TRY(validate_f32(*gate, query_values, ng.c_str()));
+    KRAKEN_TRY(validate_f32(*gate, query_values, what, " gate"));
   }
-  KRAKEN_TRY(validate_f32(output, query_values, no.c_str()));
-  const std::string nl = std::string(what) + " layer";
-  const std::string ns = std::string(what) + " start position";
-  const std::string nt = std::string(what) + " tokens";
-  const std::string nc = std::string(what) + " capacity";
-  const std::string nh = std::string(what) + " heads";
-  const std::string nkv = std::string(what) + " kv_heads";
-  const std::string nd = std::string(what) + " head_dim";
-  const std::string ngr = std::string(what) + " group";
-  KRAKEN_TRY(check_u32(layer, nl.c_str()));
-  KRAKEN_TRY(check_u32(start_position, ns.c_str()));
-  KRAKEN_TRY(check_u32(tokens, nt.c_str()));
-  KRAKEN_TRY(check_u32(capacity_tokens, nc.c_str()));
-  KRAKEN_TRY(check_u32(heads, nh.c_str()));
-  KRAKEN_TRY(check_u32(kv_heads, nkv.c_str()));
-  KRAKEN_TRY(check_u32(head_dim, nd.c_str()));
-  KRAKEN_TRY(check_u32(heads / kv_heads, ngr.c_str()));
+  KRAKEN_TRY(validate_f32(output, query_values, what, " output"));
+  KRAKEN_TRY(check_u32(layer, what, " layer"));
+  KRAKEN_TRY(check_u32(start_position, what, " start position"));
+  KRAKEN_TRY(check_u32(tokens, what, " tokens"));
+  KRAKEN_TRY(check_u32(capacity_tokens, what, " capacity"));
+  KRAKEN_TRY(check_u32(heads, what, " heads"));
+  KRAKEN_TRY(check_u32(kv_heads, what, " kv_heads"));
+  KRAKEN_TRY(check_u32(head_dim, what, " head_dim"));
+  KRAKEN_TRY(check_u32(heads / kv_heads, what, " group"));
 
   AttentionArgs a{};
   a.query = static_cast<const float*>(query.data);
@@ -135,7 +122,7 @@ int attention_entry(kraken_hip_context* ctx, const char* what, bool kv_f16,
     a.query_f16 = query.data;
   }
   if (no_alloc && need > kNoAllocScratchBytes) {
-    return invalid(w + " needs " + std::to_string(need) +
+    return invalid(w() + " needs " + std::to_string(need) +
                    " bytes of split partials; the allocation-free entry point has " +
                    std::to_string(kNoAllocScratchBytes));
   }
@@ -156,7 +143,7 @@ int attention_entry(kraken_hip_context* ctx, const char* what, bool kv_f16,
     float* q32 = reinterpret_cast<float*>(static_cast<char*>(workspace) + query_offset);
     const hipError_t ec = launch_f16_to_f32(query.data, q32, query_values, ctx->stream);
     if (ec != hipSuccess) {
-      return internal(w + " launch failed: " + hipGetErrorString(ec));
+      return internal(w() + " launch failed: " + hipGetErrorString(ec));
     }
     a.query = q32;
     workspace_bytes = query_offset;
@@ -166,9 +153,9 @@ int attention_entry(kraken_hip_context* ctx, const char* what, bool kv_f16,
               : launch_attention_decode(a, ctx->cu_count, workspace, workspace_bytes,
                                         ctx->stream);
   if (e != hipSuccess) {
-    return internal(w + " launch failed: " + hipGetErrorString(e));
+    return internal(w() + " launch failed: " + hipGetErrorString(e));
   }
-  return finish_launch(ctx, (w + " command failed: ").c_str());
+  return finish_launch(ctx, "HIP ", what, " command failed: ");
 }
 
 // gated_delta_net_f32_batched_in_place_at host side (mps_backend.mm:8517-8600).
@@ -180,41 +167,40 @@ int gdn_entry(kraken_hip_context* ctx, const char* what, const kraken_buffer& qu
               const kraken_buffer* ssm_a, const kraken_buffer* z, const kraken_buffer* norm_w,
               float eps) {
   KRAKEN_TRY(check_context(ctx));
-  const std::string w = std::string("HIP ") + what;
+  const auto w = [what] { return std::string("HIP ") + what; };
   if (tokens == 0 || key_heads == 0 || value_heads == 0 || head_dim == 0) {
-    return invalid(w + " dimensions must be positive");
+    return invalid(w() + " dimensions must be positive");
   }
   if (value_heads % key_heads != 0) {
-    return invalid(w + " value heads must repeat key heads");
+    return invalid(w() + " value heads must repeat key heads");
   }
   if (head_dim > 256u) {
-    return invalid(w + " head_dim exceeds 256");
+    return invalid(w() + " head_dim exceeds 256");
   }
   size_t kvpt = 0, vvpt = 0, key_values = 0, value_values = 0, gate_values = 0, state_values = 0;
   if (!checked_mul(key_heads, head_dim, kvpt) || !checked_mul(value_heads, head_dim, vvpt) ||
       !checked_mul(tokens, kvpt, key_values) || !checked_mul(tokens, vvpt, value_values) ||
       !checked_mul(tokens, value_heads, gate_values) ||
       !checked_mul(vvpt, head_dim, state_values)) {
-    return invalid(w + " value count overflow");
+    return invalid(w() + " value count overflow");
   }
-  const std::string base(what);
-  KRAKEN_TRY(validate_f32(query, key_values, (base + " query").c_str()));
-  KRAKEN_TRY(validate_f32(key, key_values, (base + " key").c_str()));
-  KRAKEN_TRY(validate_f32(value, value_values, (base + " value").c_str()));
-  KRAKEN_TRY(validate_f32(gate, gate_values, (base + " gate").c_str()));
-  KRAKEN_TRY(validate_f32(beta, gate_values, (base + " beta").c_str()));
+  KRAKEN_TRY(validate_f32(query, key_values, what, " query"));
+  KRAKEN_TRY(validate_f32(key, key_values, what, " key"));
+  KRAKEN_TRY(validate_f32(value, value_values, what, " value"));
+  KRAKEN_TRY(validate_f32(gate, gate_values, what, " gate"));
+  KRAKEN_TRY(validate_f32(beta, gate_values, what, " beta"));
   if (dt_bias != nullptr) {
-    KRAKEN_TRY(validate_f32(*dt_bias, value_heads, (base + " dt bias").c_str()));
-    KRAKEN_TRY(validate_f32(*ssm_a, value_heads, (base + " ssm a").c_str()));
-    KRAKEN_TRY(validate_f32(*z, value_values, (base + " z").c_str()));
-    KRAKEN_TRY(validate_f32(*norm_w, head_dim, (base + " norm weight").c_str()));
+    KRAKEN_TRY(validate_f32(*dt_bias, value_heads, what, " dt bias"));
+    KRAKEN_TRY(validate_f32(*ssm_a, value_heads, what, " ssm a"));
+    KRAKEN_TRY(validate_f32(*z, value_values, what, " z"));
+    KRAKEN_TRY(validate_f32(*norm_w, head_dim, what, " norm weight"));
   }
-  KRAKEN_TRY(validate_f32_region(state, state_offset, state_values, (base + " state").c_str()));
-  KRAKEN_TRY(validate_f32(output, value_values, (base + " output").c_str()));
-  KRAKEN_TRY(check_u32(tokens, (base + " tokens").c_str()));
-  KRAKEN_TRY(check_u32(key_heads, (base + " key_heads").c_str()));
-  KRAKEN_TRY(check_u32(value_heads, (base + " value_heads").c_str()));
-  KRAKEN_TRY(check_u32(head_dim, (base + " head_dim").c_str()));
+  KRAKEN_TRY(validate_f32_region(state, state_offset, state_values, what, " state"));
+  KRAKEN_TRY(validate_f32(output, value_values, what, " output"));
+  KRAKEN_TRY(check_u32(tokens, what, " tokens"));
+  KRAKEN_TRY(check_u32(key_heads, what, " key_heads"));
+  KRAKEN_TRY(check_u32(value_heads, what, " value_heads"));
+  KRAKEN_TRY(check_u32(head_dim, what, " head_dim"));
   KRAKEN_TRY(begin_launch(ctx));
   GdnArgs a{};
   a.query = static_cast<const float*>(query.data);
@@ -239,9 +225,9 @@ int gdn_entry(kraken_hip_context* ctx, const char* what, const kraken_buffer& qu
   const hipError_t e = launch_gated_delta_net(a, ctx->cu_count, ctx->workspace,
                                               ctx->workspace_bytes, ctx->stream);
   if (e != hipSuccess) {
-    return internal(w + " launch failed: " + hipGetErrorString(e));
+    return internal(w() + " launch failed: " + hipGetErrorString(e));
   }
-  return finish_launch(ctx, (w + " command failed: ").c_str());
+  return finish_launch(ctx, "HIP ", what, " command failed: ");
 }
 
 // qk_norm_f32_f32_batched / qwen35_norm_gated_f32_in_place host side

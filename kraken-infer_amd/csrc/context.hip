@@ -67,19 +67,16 @@ int begin_launch(kraken_hip_context* ctx) {
   return KRAKEN_OK;
 }
 
-int finish_launch(kraken_hip_context* ctx, const char* error_prefix) {
+int finish_launch(kraken_hip_context* ctx, const char* a, const char* b, const char* c) {
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) {
-    return internal(std::string(error_prefix) + hip_message(e));
+  if (e == hipSuccess && !ctx->graph_active) {
+    e = hipStreamSynchronize(ctx->stream);
   }
-  if (ctx->graph_active) {
-    return KRAKEN_OK;
-  }
-  e = hipStreamSynchronize(ctx->stream);
-  if (e != hipSuccess) {
-    return internal(std::string(error_prefix) + hip_message(e));
-  }
-  return KRAKEN_OK;
+  return e == hipSuccess ? KRAKEN_OK : internal(std::string(a) + b + c + hip_message(e));
+}
+
+int finish_launch(kraken_hip_context* ctx, const char* error_prefix) {
+  return finish_launch(ctx, error_prefix, "", "");
 }
 
 int ensure_workspace(kraken_hip_context* ctx, size_t bytes) {

@@ -62,6 +62,8 @@ int begin_launch(kraken_hip_context* ctx);
 // After enqueueing: checks the launch and, outside a graph, waits for the stream
 // (finish_command_buffer, mps_backend.mm:4416-4428).
 int finish_launch(kraken_hip_context* ctx, const char* error_prefix);
+// The same with the prefix in three parts, joined only for an error's message.
+int finish_launch(kraken_hip_context* ctx, const char* a, const char* b, const char* c);
 
 // Ensures ctx->workspace holds at least `bytes`.  A larger workspace is a new
 // allocation; the old one stays valid (and allocated) until the context is
@@ -105,8 +107,26 @@ int check_u32(size_t value, const char* name);
 // validate_f32/f16/i32_buffer: byte count overflow, "not initialized", "too small".
 int validate_buffer(const kraken_buffer& buffer, size_t values, size_t element_bytes,
                     const char* name);
+// check_u32 and validate_buffer with the name in two parts, joined only where the
+// check fails: the joined names cost a call of many operands 1 us.
+inline int check_u32(size_t value, const char* base, const char* part) {
+  return fits_u32(value) ? KRAKEN_OK : check_u32(value, (std::string(base) + part).c_str());
+}
+inline int validate_buffer(const kraken_buffer& buffer, size_t values, size_t element_bytes,
+                           const char* base, const char* part) {
+  size_t bytes = 0;
+  if (checked_mul(values, element_bytes, bytes) && buffer.data != nullptr &&
+      buffer.byte_size >= bytes) {
+    return KRAKEN_OK;
+  }
+  return validate_buffer(buffer, values, element_bytes, (std::string(base) + part).c_str());
+}
 inline int validate_f32(const kraken_buffer& b, size_t values, const char* name) {
   return validate_buffer(b, values, sizeof(float), name);
+}
+inline int validate_f32(const kraken_buffer& b, size_t values, const char* base,
+                        const char* part) {
+  return validate_buffer(b, values, sizeof(float), base, part);
 }
 inline int validate_f16(const kraken_buffer& b, size_t values, const char* name) {
   return validate_buffer(b, values, sizeof(uint16_t), name);
@@ -118,6 +138,15 @@ inline int validate_i32(const kraken_buffer& b, size_t values, const char* name)
 // validate_f32_buffer_region: [offset, offset+values) must fit; returns status.
 int validate_f32_region(const kraken_buffer& b, size_t offset, size_t values,
                         const char* name);
+inline int validate_f32_region(const kraken_buffer& b, size_t offset, size_t values,
+                               const char* base, const char* part) {
+  size_t end = 0, bytes = 0;
+  if (b.data != nullptr && checked_add(offset, values, end) &&
+      checked_mul(end, sizeof(float), bytes) && b.byte_size >= bytes) {
+    return KRAKEN_OK;
+  }
+  return validate_f32_region(b, offset, values, (std::string(base) + part).c_str());
+}
 
 // strided_f32_region_end (mps_backend.mm:4203-4231): end element of a strided
 // row range; invalid argument on zero rows/row_size, stride < row_size, overflow.

@@ -214,6 +214,38 @@ def as_buffer(obj) -> KrakenBuffer:
     raise TypeError(f"cannot make a kraken_buffer from {type(obj)}")
 
 
+# name -> (C function, its argument count, which of them are buffers), so that a
+# call does not look these up again.
+_calls = {}
+
+
+def _bind(name: str):
+    full = "kraken_hip_" + name
+    diag = full in DIAG_SIGNATURES
+    types = DIAG_SIGNATURES[full] if diag else SIGNATURES[full]
+    fn = getattr(diag_lib() if diag else lib(), full)
+    entry = (fn, len(types), tuple(i for i, t in enumerate(types) if t is KrakenBuffer))
+    _calls[name] = entry
+    return entry
+
+
+_EMPTY = KrakenBuffer(None, 0)
+# Array types of the per-matrix arguments of the multi-matrix entries, by length.
+_U32S = [ctypes.c_uint32 * n for n in range(5)]
+_SIZES = [ctypes.c_size_t * n for n in range(5)]
+_BUFFERS = [KrakenBuffer * n for n in range(5)]
+
+
+def _array(types, element, n, values):
+    """A ctypes array of n elements from at most n values."""
+    return (types[n] if n < len(types) else element * n)(*values)
+
+
+def _views(buffers):
+    return [b if type(b) is KrakenBuffer else _EMPTY if b is None else as_buffer(b)
+            for b in buffers]
+
+
 class DeviceBuffer:
     """Device allocation owned through the context (make_buffer / free_buffer)."""
 
@@ -283,34 +315,33 @@ class Context:
 
     def status(self, name: str, *args) -> int:
         """Calls kraken_hip_<name> and returns its status code."""
-        full = "kraken_hip_" + name
-        diag = full in DIAG_SIGNATURES
-        fn = getattr(diag_lib() if diag else lib(), full)
-        types = DIAG_SIGNATURES[full] if diag else SIGNATURES[full]
-        conv = [as_buffer(a) if t is KrakenBuffer else a for a, t in zip(args, types)]
-        return fn(self.handle, *conv)
+        fn, count, buffers = _calls.get(name) or _bind(name)
+        args = list(args[:count])
+        for i in buffers:
+            if i >= len(args):
+                break  # too few: ctypes says so
+            a = args[i]
+            if type(a) is not KrakenBuffer:
+                args[i] = _EMPTY if a is None else as_buffer(a)
+        return fn(self.handle, *args)
 
     def call(self, name: str, *args):
         code = self.status(name, *args)
-        if code != OK and "kraken_hip_" + name in DIAG_SIGNATURES:
-            raise KrakenError(code, diag_lib().kraken_hip_diag_last_error().decode(), name)
-        self._check(name, code)
-
-    def __getattr__(self, name):
-        if "kraken_hip_" + name in SIGNATURES or "kraken_hip_" + name in DIAG_SIGNATURES:
-            return lambda *args: self.call(name, *args)
-        raise AttributeError(name)
+        if code != OK:
+            if "kraken_hip_" + name in DIAG_SIGNATURES:
+                raise KrakenError(code, diag_lib().kraken_hip_diag_last_error().decode(), name)
+            self._check(name, code)
 
     def kquant_matvec_multi(self, ggml_types, weights, rows, cols, input, norm_weight, eps,
                             up, residuals, outputs):
         """kraken_hip_kquant_matvec_multi_f32 with Python sequences for the
         per-matrix arrays (residual entries may be None)."""
         n = len(weights)
-        types = (ctypes.c_uint32 * n)(*ggml_types)
-        ws = (KrakenBuffer * n)(*[as_buffer(w) for w in weights])
-        rs = (ctypes.c_size_t * n)(*rows)
-        res = (KrakenBuffer * n)(*[as_buffer(r) for r in residuals])
-        outs = (KrakenBuffer * n)(*[as_buffer(o) for o in outputs])
+        types = _array(_U32S, ctypes.c_uint32, n, ggml_types)
+        ws = _array(_BUFFERS, KrakenBuffer, n, _views(weights))
+        rs = _array(_SIZES, ctypes.c_size_t, n, rows)
+        res = _array(_BUFFERS, KrakenBuffer, n, _views(residuals))
+        outs = _array(_BUFFERS, KrakenBuffer, n, _views(outputs))
         self.call("kquant_matvec_multi_f32", n, types, ws, rs, cols, input, norm_weight, eps, up,
                   res, outs)
 
@@ -318,10 +349,10 @@ class Context:
         """kraken_hip_kquant_matmul_multi_f32 with Python sequences for the
         per-matrix arrays."""
         n = len(weights)
-        types = (ctypes.c_uint32 * n)(*ggml_types)
-        ws = (KrakenBuffer * n)(*[as_buffer(w) for w in weights])
-        rs = (ctypes.c_size_t * n)(*rows)
-        outs = (KrakenBuffer * n)(*[as_buffer(o) for o in outputs])
+        types = _array(_U32S, ctypes.c_uint32, n, ggml_types)
+        ws = _array(_BUFFERS, KrakenBuffer, n, _views(weights))
+        rs = _array(_SIZES, ctypes.c_size_t, n, rows)
+        outs = _array(_BUFFERS, KrakenBuffer, n, _views(outputs))
         self.call("kquant_matmul_multi_f32", n, types, ws, rs, cols, tokens, input, outs)
 
     def kquant_matvec_multi_conv(self, ggml_types, weights, rows, cols, input, norm_weight, eps,
@@ -329,10 +360,10 @@ class Context:
         """kraken_hip_kquant_matvec_multi_conv_f32 with Python sequences for the
         per-matrix arrays."""
         n = len(weights)
-        types = (ctypes.c_uint32 * n)(*ggml_types)
-        ws = (KrakenBuffer * n)(*[as_buffer(w) for w in weights])
-        rs = (ctypes.c_size_t * n)(*rows)
-        outs = (KrakenBuffer * n)(*[as_buffer(o) for o in outputs])
+        types = _array(_U32S, ctypes.c_uint32, n, ggml_types)
+        ws = _array(_BUFFERS, KrakenBuffer, n, _views(weights))
+        rs = _array(_SIZES, ctypes.c_size_t, n, rows)
+        outs = _array(_BUFFERS, KrakenBuffer, n, _views(outputs))
         self.call("kquant_matvec_multi_conv_f32", n, types, ws, rs, cols, input, norm_weight, eps,
                   outs, conv_pool, conv_offset, conv_weights, conv_kernel)
 
@@ -355,6 +386,21 @@ class Context:
 
     def abort_graph(self):
         lib().kraken_hip_abort_graph(self.handle)
+
+
+def _entry_method(name):
+    def method(self, *args):
+        self.call(name, *args)
+
+    method.__name__ = name
+    return method
+
+
+# Every entry point as a Context method (Context's own methods stay).
+for _full in (*SIGNATURES, *DIAG_SIGNATURES):
+    _name = _full[len("kraken_hip_"):]
+    if not hasattr(Context, _name):
+        setattr(Context, _name, _entry_method(_name))
 
 
 def _f32(a) -> np.ndarray:
