@@ -203,12 +203,19 @@ inline bool env_is(const char* name, const char* value) {
 }  // namespace bench_detail
 
 // The GDN kernel this backend runs for the shape (KRAKEN_GDN_PREFILL overrides
-// the head_dim-128 multi-token choice).
-inline std::string gdn_dispatch_name(std::size_t tokens, std::size_t head_dim) {
+// the head_dim-128 multi-token choice): from 64 tokens on the chunked kernels, past
+// 160 tokens for up to 32 value heads and past 96 for up to 64.
+inline std::string gdn_dispatch_name(std::size_t tokens, std::size_t head_dim,
+                                     std::size_t value_heads = 16U) {
   if (head_dim != 128U || bench_detail::env_is("KRAKEN_GDN_PREFILL", "generic")) {
     return "generic_batched_gdn";
   }
-  if (tokens >= 64U && !bench_detail::env_is("KRAKEN_GDN_PREFILL", "sequential")) {
+  const std::size_t recurrence = bench_detail::env_is("KRAKEN_GDN_PREFILL", "chunked") ? 0U
+                                 : value_heads <= 32U                                  ? 160U
+                                 : value_heads <= 64U                                  ? 96U
+                                                                                       : 0U;
+  if (tokens >= 64U && tokens > recurrence &&
+      !bench_detail::env_is("KRAKEN_GDN_PREFILL", "sequential")) {
     return "chunked_wy";
   }
   return "recurrence_128";
@@ -526,7 +533,8 @@ inline hip::Result<GdnBenchResult> benchmark_gdn(const GdnBenchConfig& config) {
   const double total_seconds = seconds.value();
   const auto timed = static_cast<double>(config.timed_iterations);
   GdnBenchResult result;
-  result.dispatch = gdn_dispatch_name(config.tokens, config.head_dim);
+  result.dispatch =
+    gdn_dispatch_name(config.tokens, config.head_dim, config.value_heads);
   result.tokens = config.tokens;
   result.key_heads = config.key_heads;
   result.value_heads = config.value_heads;

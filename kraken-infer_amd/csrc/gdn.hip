@@ -27,8 +27,9 @@ namespace {
 
 // KRAKEN_GDN_PREFILL selects the multi-token kernel for head_dim 128:
 // "sequential" the LDS-staged recurrence, "generic" the generic recurrence
-// kernel; unset, the chunked (WY) kernels of gdn_chunked.hip run.  Used to
-// compare the three on the same inputs.
+// kernel, "chunked" the chunked (WY) kernels of gdn_chunked.hip from 64 tokens on;
+// unset, the rule in gdn_chunked_supported.  Used to compare the three on the same
+// inputs.
 bool gdn_prefill_disabled() {
   const char* v = std::getenv("KRAKEN_GDN_PREFILL");
   return v != nullptr && std::strcmp(v, "generic") == 0;
@@ -292,23 +293,47 @@ __device__ __forceinline__ float half_sum32(float x) {
 // 16 workgroups per head), but the per-token inputs come from LDS: the
 // workgroup stages kGdnChunk tokens of k, q (the whole 128-wide rows), its 8
 // values of v, and the per-token decay exp(g) and beta (prepared once per token
-// here rather than per lane) into one of two LDS buffers while the other is
-// consumed, so no token waits on global memory.  The per-token arithmetic is
+// here rather than per lane) into LDS, with the next kGdnChunk tokens on their way
+// into registers, so no token waits on global memory.  The per-token arithmetic is
 // the reference's, in its order: S *= exp(g); sk = S.k; delta = (v - sk) beta;
 // S += k delta; y = S.q / sqrt(D).  The host checks 16-byte alignment of
 // q/k/v/state and value_heads * 128 % 4 == 0 (always true for D = 128).
+//
+// With 16 heads a wave has its SIMD to itself, so what bounds a token is the number
+// of its instructions: 85 when a token read its own inputs, reduced its own y and
+// stored it.  Four tokens at a time share the input reads (in flight a group ahead,
+// no copies), the y reductions (quad_sums4) and the store.  One LDS buffer instead
+// of two lets two workgroups share a CU, for which 32 heads are enough.  45 tokens,
+// 16 heads, with the conv prologue and the norm: 21.0 -> 18.2 us; 63 tokens, 32
+// heads: 39.3 -> 23.0 us; same bits.
 constexpr int kGdnChunk = 64;
 
+// half_sum32 of four values at once: lane l ends with the sum of value
+// quad_value(l), in half_sum32's order of additions.  The first two steps give
+// each lane of a quad one of the values; odd quads hold them mirrored, so that the
+// two mirror steps meet their own.
+__device__ __forceinline__ int quad_value(int lane) { return (lane & 3) ^ ((lane & 4) ? 3 : 0); }
+
+__device__ __forceinline__ float quad_sums4(const float y[4], bool b0, bool b1) {
+  const float lo = (b0 ? y[1] : y[0]) + dpp<kDppQuadXor1>(b0 ? y[0] : y[1]);
+  const float hi = (b0 ? y[3] : y[2]) + dpp<kDppQuadXor1>(b0 ? y[2] : y[3]);
+  float x = (b1 ? hi : lo) + dpp<kDppQuadXor2>(b1 ? lo : hi);
+  x += dpp<kDppRowHalfMirror>(x);
+  x += dpp<kDppRowMirror>(x);
+  return xor16_sum(x);
+}
+
 template <bool kPrepare>
-__global__ __launch_bounds__(256) void gdn_prefill_kernel(GdnParams p) {
+__global__ __launch_bounds__(256, 2) void gdn_prefill_kernel(GdnParams p) {
   constexpr uint32_t D = 128;
   constexpr int TC = kGdnChunk;
   constexpr int kRows = 8;
-  __shared__ float4 s_k[2][TC][D / 4];
-  __shared__ float4 s_q[2][TC][D / 4];
-  __shared__ float s_v[2][TC][kRows];
-  __shared__ float s_decay[2][TC];
-  __shared__ float s_beta[2][TC];
+  constexpr int kVStride = TC + 4;  // floats: a row's four tokens are one 16-byte read
+  __shared__ float4 s_k[TC][D / 4];
+  __shared__ float4 s_q[TC][D / 4];
+  __shared__ __attribute__((aligned(16))) float s_v[kRows][kVStride];
+  __shared__ __attribute__((aligned(16))) float s_decay[TC];
+  __shared__ __attribute__((aligned(16))) float s_beta[TC];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -363,73 +388,108 @@ __global__ __launch_bounds__(256) void gdn_prefill_kernel(GdnParams p) {
       }
     }
   };
-  auto store_chunk = [&](int buf) {
+  auto store_chunk = [&]() {
 #pragma unroll
     for (int i = 0; i < TC * 32 / 256; ++i) {
       const uint32_t idx = tid + 256u * i;
-      s_k[buf][idx >> 5][idx & 31u] = kr[i];
-      s_q[buf][idx >> 5][idx & 31u] = qr[i];
+      s_k[idx >> 5][idx & 31u] = kr[i];
+      s_q[idx >> 5][idx & 31u] = qr[i];
     }
     if (tid < 2 * TC) {
-      *reinterpret_cast<float4*>(&s_v[buf][tid >> 1][4 * (tid & 1)]) = vr;
+      const int t = tid >> 1, r = 4 * (tid & 1);
+      s_v[r][t] = vr.x;
+      s_v[r + 1][t] = vr.y;
+      s_v[r + 2][t] = vr.z;
+      s_v[r + 3][t] = vr.w;
     } else if (tid < 3 * TC) {
-      s_decay[buf][tid - 2 * TC] = dr;
-      s_beta[buf][tid - 2 * TC] = br;
+      s_decay[tid - 2 * TC] = dr;
+      s_beta[tid - 2 * TC] = br;
     }
   };
 
+  struct Group {  // four tokens' inputs
+    float4 k[4], q[4], v, decay, beta;
+  };
+  auto read_group = [&](int g, Group& x) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      x.k[j] = s_k[4 * g + j][c4];
+      x.q[j] = s_q[4 * g + j][c4];
+    }
+    x.v = *reinterpret_cast<const float4*>(&s_v[lrow][4 * g]);
+    x.decay = *reinterpret_cast<const float4*>(&s_decay[4 * g]);
+    x.beta = *reinterpret_cast<const float4*>(&s_beta[4 * g]);
+  };
+  // One token; returns this lane's part of y.
+  auto step = [&](const float4& k, const float4& q, float v, float decay,
+                  float b) __attribute__((always_inline)) {
+    s.x *= decay;
+    s.y *= decay;
+    s.z *= decay;
+    s.w *= decay;
+    float sk = fmaf(s.w, k.w, fmaf(s.z, k.z, fmaf(s.y, k.y, s.x * k.x)));
+    sk = half_sum32(sk);
+    const float delta = (v - sk) * b;
+    s.x = fmaf(k.x, delta, s.x);
+    s.y = fmaf(k.y, delta, s.y);
+    s.z = fmaf(k.z, delta, s.z);
+    s.w = fmaf(k.w, delta, s.w);
+    return fmaf(s.w, q.w, fmaf(s.z, q.z, fmaf(s.y, q.y, s.x * q.x)));
+  };
+  const int yt = quad_value(c4);  // the token of a group whose y this lane ends with
+  const bool b0 = (yt & 1) != 0, b1 = (yt & 2) != 0;
+
   load_chunk(0);
-  store_chunk(0);
+  store_chunk();
   __syncthreads();
   for (uint32_t c = 0; c < chunks; ++c) {
-    const int buf = (int)(c & 1u);
     if (c + 1 < chunks) {
       load_chunk(c + 1);  // lands while this chunk computes
     }
     const uint32_t tb = c * TC;
     const int n = (int)min((uint32_t)TC, tokens - tb);
-    float* out = p.output + ((size_t)tb * p.value_heads + h) * D + row;
     const size_t out_stride = (size_t)p.value_heads * D;
-    float4 k = s_k[buf][0][c4];
-    float4 q = s_q[buf][0][c4];
-    float v = s_v[buf][0][lrow];
-    float decay = s_decay[buf][0];
-    float b = s_beta[buf][0];
-    for (int t = 0; t < n; ++t) {
-      // Next token's inputs (clamped at the chunk end) before this token's math.
-      const int tn = t + 1 < n ? t + 1 : t;
-      const float4 k_n = s_k[buf][tn][c4];
-      const float4 q_n = s_q[buf][tn][c4];
-      const float v_n = s_v[buf][tn][lrow];
-      const float decay_n = s_decay[buf][tn];
-      const float b_n = s_beta[buf][tn];
-
-      s.x *= decay;
-      s.y *= decay;
-      s.z *= decay;
-      s.w *= decay;
-      float sk = fmaf(s.w, k.w, fmaf(s.z, k.z, fmaf(s.y, k.y, s.x * k.x)));
-      sk = half_sum32(sk);
-      const float delta = (v - sk) * b;
-      s.x = fmaf(k.x, delta, s.x);
-      s.y = fmaf(k.y, delta, s.y);
-      s.z = fmaf(k.z, delta, s.z);
-      s.w = fmaf(k.w, delta, s.w);
-      float y = fmaf(s.w, q.w, fmaf(s.z, q.z, fmaf(s.y, q.y, s.x * q.x)));
-      y = half_sum32(y);
-      if (c4 == 0) {
-        out[(size_t)t * out_stride] = y * p.scale;
+    // Lanes 0 .. 3 of a row store the y of tokens 0 .. 3 of a group.
+    float* out = p.output + ((size_t)(tb + yt) * p.value_heads + h) * D + row;
+    auto group = [&](int g, const Group& x) __attribute__((always_inline)) {
+      float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      if (4 * g + 4 <= n) {
+        y[0] = step(x.k[0], x.q[0], x.v.x, x.decay.x, x.beta.x);
+        y[1] = step(x.k[1], x.q[1], x.v.y, x.decay.y, x.beta.y);
+        y[2] = step(x.k[2], x.q[2], x.v.z, x.decay.z, x.beta.z);
+        y[3] = step(x.k[3], x.q[3], x.v.w, x.decay.w, x.beta.w);
+      } else {
+        y[0] = step(x.k[0], x.q[0], x.v.x, x.decay.x, x.beta.x);
+        if (4 * g + 1 < n) {
+          y[1] = step(x.k[1], x.q[1], x.v.y, x.decay.y, x.beta.y);
+        }
+        if (4 * g + 2 < n) {
+          y[2] = step(x.k[2], x.q[2], x.v.z, x.decay.z, x.beta.z);
+        }
       }
-      k = k_n;
-      q = q_n;
-      v = v_n;
-      decay = decay_n;
-      b = b_n;
+      const float sum = quad_sums4(y, b0, b1);
+      if (c4 < 4 && 4 * g + yt < n) {
+        out[(size_t)(4 * g) * out_stride] = sum * p.scale;
+      }
+    };
+    // The next group's inputs (clamped at the chunk's end) are read before a
+    // group's math.
+    const int groups = (n + 3) / 4;
+    Group x[2];
+    read_group(0, x[0]);
+    for (int g = 0; g < groups; g += 2) {
+      read_group(min(g + 1, groups - 1), x[1]);
+      group(g, x[0]);
+      read_group(min(g + 2, groups - 1), x[0]);
+      if (g + 1 < groups) {
+        group(g + 1, x[1]);
+      }
     }
     if (c + 1 < chunks) {
-      store_chunk(buf ^ 1);  // buffer buf ^ 1 was last read before the previous barrier
+      __syncthreads();  // every wave is done with this chunk's inputs
+      store_chunk();
+      __syncthreads();
     }
-    __syncthreads();
   }
   *reinterpret_cast<float4*>(srow) = s;
 }

@@ -816,8 +816,23 @@ bool gdn_chunked_supported(const GdnArgs& a) {
   }
   const bool aligned = ((uintptr_t)a.query | (uintptr_t)a.key | (uintptr_t)a.value |
                         (uintptr_t)a.state | (uintptr_t)a.output) % 16u == 0;
-  return a.seq_state_offsets == nullptr && a.head_dim == (uint32_t)kDim && aligned &&
-         a.tokens >= (uint32_t)kC;
+  if (a.seq_state_offsets != nullptr || a.head_dim != (uint32_t)kDim || !aligned ||
+      a.tokens < (uint32_t)kC) {
+    return false;
+  }
+  // The recurrence costs a fixed time per token (more where its 16 workgroups per
+  // head exceed two per CU), the three launches of the chunked form a fixed time
+  // first.  Measured with the conv prologue and the norm, us, recurrence / chunked:
+  //   heads   64 tokens   96 tokens   128 tokens  160 tokens  192 tokens  256 tokens
+  //     16    21.0 / 35   27.7 / 40   32.3 / 41   37.2 / 43   42.6 / 46   52.2 / 46
+  //     32    23.2 / 37   30.8 / 43   37.3 / 46   43.8 / 46   48.5 / 46   59.1 / 49
+  //     48    31.8 / 42   42.6 / 49   52.6 / 48
+  //     64    35.0 / 44   47.6 / 49   58.0 / 50
+  if (v != nullptr && std::strcmp(v, "chunked") == 0) {
+    return true;
+  }
+  const uint32_t recurrence = a.value_heads <= 32u ? 160u : (a.value_heads <= 64u ? 96u : 0u);
+  return a.tokens > recurrence;
 }
 
 size_t gdn_chunked_workspace_bytes(const GdnArgs& a) {
