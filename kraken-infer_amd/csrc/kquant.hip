@@ -1751,66 +1751,90 @@ __device__ __forceinline__ bool better(float v, uint32_t i, float bv, uint32_t b
   return v > bv || (v == bv && i < bi);
 }
 
-// Candidate of [begin, end) of `values`, reduced over a 256-thread workgroup.
-// `with_sum` adds the range's sum of exp(v - max).
-__device__ ArgCand block_candidate(const float* values, uint64_t begin, uint64_t end,
-                                   uint32_t size_marker, bool with_sum) {
-  __shared__ float s_v[256];
-  __shared__ uint32_t s_i[256];
-  __shared__ float s_s[256];
-  const int tid = threadIdx.x;
-  float bv = -INFINITY;
-  uint32_t bi = size_marker;
-  for (uint64_t i = begin + tid; i < end; i += 256) {
-    const float v = values[i];
-    if (better(v, (uint32_t)i, bv, bi)) {
+// The best (value, first index) and the sum over a 256-thread workgroup, in every
+// thread: lane exchanges within a wave, one barrier for the four waves.  s_v, s_i
+// and s_s hold four values each, used once per kernel.
+__device__ __forceinline__ void block_best(float& bv, uint32_t& bi, float* s_v, uint32_t* s_i) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const float v = __shfl_xor(bv, off, 64);
+    const uint32_t i = __shfl_xor(bi, off, 64);
+    if (better(v, i, bv, bi)) {
       bv = v;
+      bi = i;
+    }
+  }
+  if ((threadIdx.x & 63) == 0) {
+    s_v[threadIdx.x >> 6] = bv;
+    s_i[threadIdx.x >> 6] = bi;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    if (better(s_v[w], s_i[w], bv, bi)) {
+      bv = s_v[w];
+      bi = s_i[w];
+    }
+  }
+}
+
+__device__ __forceinline__ float block_sum(float x, float* s_s) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    x += __shfl_xor(x, off, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    s_s[threadIdx.x >> 6] = x;
+  }
+  __syncthreads();
+  return (s_s[0] + s_s[1]) + (s_s[2] + s_s[3]);
+}
+
+// exp(v - max) as a term of a range's sum.  A range whose values are all -inf or
+// NaN has max == -inf; its -inf entries count 0 (they add exp(-inf) to any finite
+// overall maximum) and its NaNs stay NaN, so the merged sum is what one pass
+// would give.
+__device__ __forceinline__ float exp_term(float v, float max) {
+  return v == -INFINITY && max == -INFINITY ? 0.0f : expf(v - max);
+}
+
+// Phase 1: workgroup g takes values [g * 256 kPer, (g + 1) * 256 kPer), each read
+// once and kept in registers.  Bound by latency: 248320 values in 61 workgroups of
+// 4096, read twice with 16 barriers between, took 9.8 us; 243 of 1024, two
+// barriers: 4.6 us.
+template <int kPer>
+__global__ __launch_bounds__(256) void argmax_partial_kernel(const float* values, uint64_t size,
+                                                             bool with_sum, ArgCand* cands) {
+  __shared__ float s_v[4], s_s[4];
+  __shared__ uint32_t s_i[4];
+  const uint64_t begin = (uint64_t)blockIdx.x * (256u * kPer) + threadIdx.x;
+  float v[kPer];
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const uint64_t i = begin + 256u * j;
+    v[j] = i < size ? values[i] : -INFINITY;
+  }
+  float bv = -INFINITY;
+  uint32_t bi = (uint32_t)size;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const uint64_t i = begin + 256u * j;
+    if (i < size && better(v[j], (uint32_t)i, bv, bi)) {
+      bv = v[j];
       bi = (uint32_t)i;
     }
   }
-  s_v[tid] = bv;
-  s_i[tid] = bi;
-  __syncthreads();
-  for (int stride = 128; stride > 0; stride >>= 1) {
-    if (tid < stride && better(s_v[tid + stride], s_i[tid + stride], s_v[tid], s_i[tid])) {
-      s_v[tid] = s_v[tid + stride];
-      s_i[tid] = s_i[tid + stride];
-    }
-    __syncthreads();
-  }
-  ArgCand r{s_v[0], s_i[0], 0.0f};
+  block_best(bv, bi, s_v, s_i);
+  float sum = 0.0f;
   if (with_sum) {
-    // A range whose values are all -inf or NaN has r.value == -inf; its -inf
-    // entries count 0 (they add exp(-inf) to any finite overall maximum) and
-    // its NaNs stay NaN, so the merged sum is what one pass would give.
-    float sum = 0.0f;
-    for (uint64_t i = begin + tid; i < end; i += 256) {
-      const float v = values[i];
-      sum += (v == -INFINITY && r.value == -INFINITY) ? 0.0f : expf(v - r.value);
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      sum += begin + 256u * j < size ? exp_term(v[j], bv) : 0.0f;
     }
-    s_s[tid] = sum;
-    __syncthreads();
-    for (int stride = 128; stride > 0; stride >>= 1) {
-      if (tid < stride) {
-        s_s[tid] += s_s[tid + stride];
-      }
-      __syncthreads();
-    }
-    r.sum = s_s[0];
+    sum = block_sum(sum, s_s);
   }
-  __syncthreads();
-  return r;
-}
-
-// Phase 1: workgroup g takes [g * span, (g + 1) * span).
-__global__ __launch_bounds__(256) void argmax_partial_kernel(const float* values, uint64_t size,
-                                                             uint64_t span, bool with_sum,
-                                                             ArgCand* cands) {
-  const uint64_t begin = (uint64_t)blockIdx.x * span;
-  const uint64_t end = min(size, begin + span);
-  const ArgCand r = block_candidate(values, begin, end, (uint32_t)size, with_sum);
   if (threadIdx.x == 0) {
-    cands[blockIdx.x] = r;
+    cands[blockIdx.x] = ArgCand{bv, bi, sum};
   }
 }
 
@@ -1824,64 +1848,55 @@ __global__ __launch_bounds__(256) void argmax_final_kernel(const float* values, 
                                                            bool with_sum, bool max_above_neg_inf,
                                                            int32_t* token_out,
                                                            float* probability_out) {
-  __shared__ float s_v[256];
-  __shared__ uint32_t s_i[256];
-  __shared__ float s_s[256];
+  __shared__ float s_v[4], s_s[4];
+  __shared__ uint32_t s_i[4];
   const int tid = threadIdx.x;
-  if (cands == nullptr) {
-    const ArgCand r = block_candidate(values, 0, size, (uint32_t)size, with_sum);
-    if (tid == 0) {
-      token_out[0] = max_above_neg_inf && !(r.value > -INFINITY) ? 0 : (int32_t)r.index;
-      if (probability_out != nullptr) {
-        probability_out[0] = r.sum > 0.0f ? 1.0f / r.sum : 0.0f;
-      }
-    }
-    return;
-  }
   float bv = -INFINITY;
   uint32_t bi = (uint32_t)size;
-  for (uint32_t g = tid; g < count; g += 256) {
-    if (better(cands[g].value, cands[g].index, bv, bi)) {
-      bv = cands[g].value;
-      bi = cands[g].index;
-    }
-  }
-  s_v[tid] = bv;
-  s_i[tid] = bi;
-  __syncthreads();
-  for (int stride = 128; stride > 0; stride >>= 1) {
-    if (tid < stride && better(s_v[tid + stride], s_i[tid + stride], s_v[tid], s_i[tid])) {
-      s_v[tid] = s_v[tid + stride];
-      s_i[tid] = s_i[tid + stride];
-    }
-    __syncthreads();
-  }
-  const float gmax = s_v[0];
-  const uint32_t gidx = s_i[0];
-  if (with_sum) {
-    float sum = 0.0f;
-    for (uint32_t g = tid; g < count; g += 256) {
-      sum += cands[g].sum * expf(cands[g].value - gmax);
-    }
-    s_s[tid] = sum;
-    __syncthreads();
-    for (int stride = 128; stride > 0; stride >>= 1) {
-      if (tid < stride) {
-        s_s[tid] += s_s[tid + stride];
+  float sum = 0.0f;
+  if (cands == nullptr) {
+    for (uint64_t i = tid; i < size; i += 256) {
+      const float v = values[i];
+      if (better(v, (uint32_t)i, bv, bi)) {
+        bv = v;
+        bi = (uint32_t)i;
       }
-      __syncthreads();
     }
+    block_best(bv, bi, s_v, s_i);
+    if (with_sum) {
+      for (uint64_t i = tid; i < size; i += 256) {
+        sum += exp_term(values[i], bv);
+      }
+    }
+  } else {
+    for (uint32_t g = tid; g < count; g += 256) {
+      if (better(cands[g].value, cands[g].index, bv, bi)) {
+        bv = cands[g].value;
+        bi = cands[g].index;
+      }
+    }
+    block_best(bv, bi, s_v, s_i);
+    if (with_sum) {
+      for (uint32_t g = tid; g < count; g += 256) {
+        sum += cands[g].sum * expf(cands[g].value - bv);
+      }
+    }
+  }
+  if (with_sum) {
+    sum = block_sum(sum, s_s);
   }
   if (tid == 0) {
-    token_out[0] = max_above_neg_inf && !(gmax > -INFINITY) ? 0 : (int32_t)gidx;
+    token_out[0] = max_above_neg_inf && !(bv > -INFINITY) ? 0 : (int32_t)bi;
     if (probability_out != nullptr) {
-      probability_out[0] = s_s[0] > 0.0f ? 1.0f / s_s[0] : 0.0f;
+      probability_out[0] = sum > 0.0f ? 1.0f / sum : 0.0f;
     }
   }
 }
 
 constexpr uint64_t kArgmaxSingleMax = 16384;  // one workgroup up to this size
-constexpr uint64_t kArgmaxSpan = 4096;        // values per phase-1 workgroup
+// Values per thread of a phase-1 workgroup: 16, or 4 where that gives at most the
+// 256 candidates that phase 2 takes in one pass and the workspace holds them.
+constexpr uint64_t kArgmaxPer = 16, kArgmaxPerSmall = 4;
 
 template <int F>
 hipError_t launch_gemv_f(const GemvArgs& base, hipStream_t stream) {
@@ -2318,7 +2333,7 @@ size_t argmax_workspace_bytes(size_t size) {
   if (size <= kArgmaxSingleMax) {
     return 0;
   }
-  const size_t groups = (size + kArgmaxSpan - 1) / kArgmaxSpan;
+  const size_t groups = (size + 256u * kArgmaxPer - 1) / (256u * kArgmaxPer);
   return groups * sizeof(ArgCand);
 }
 
@@ -2331,13 +2346,22 @@ hipError_t launch_argmax(const float* values, size_t size, int32_t* token_out,
                                                token_out, probability_out);
     return hipGetLastError();
   }
-  const size_t groups = (size + kArgmaxSpan - 1) / kArgmaxSpan;
+  size_t groups = (size + 256u * kArgmaxPerSmall - 1) / (256u * kArgmaxPerSmall);
+  const bool small = groups <= 256u && workspace_bytes >= groups * sizeof(ArgCand);
+  if (!small) {
+    groups = (size + 256u * kArgmaxPer - 1) / (256u * kArgmaxPer);
+  }
   if (workspace == nullptr || workspace_bytes < groups * sizeof(ArgCand)) {
     return hipErrorInvalidValue;
   }
   ArgCand* cands = static_cast<ArgCand*>(workspace);
-  argmax_partial_kernel<<<dim3((uint32_t)groups), 256, 0, stream>>>(values, size, kArgmaxSpan,
-                                                                    with_sum, cands);
+  if (small) {
+    argmax_partial_kernel<kArgmaxPerSmall>
+      <<<dim3((uint32_t)groups), 256, 0, stream>>>(values, size, with_sum, cands);
+  } else {
+    argmax_partial_kernel<kArgmaxPer>
+      <<<dim3((uint32_t)groups), 256, 0, stream>>>(values, size, with_sum, cands);
+  }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     return e;
