@@ -24,7 +24,6 @@ struct DecodeParams {
   float* part_ml;  // [tokens][kv_heads][splits][G][2]
   uint32_t layer, start_position, tokens, capacity_tokens, heads, kv_heads;
   uint32_t keys_per_split, splits;
-  bool rows;  // a several-token kernel (attention_rows.hip, attention_rows_f32.hip)
   float scale_log2;
   // Ragged multi-sequence mode (see AttentionArgs): per-token K/V element
   // offsets and positions, and the pools' element count.
@@ -34,6 +33,9 @@ struct DecodeParams {
   // Ragged mode: dense work list, one item per workgroup (blockIdx.x):
   // {token, kv_head << 16 | split}, token 0xffffffff past the last item.
   const uint2* work_items;
+  // A several-token kernel (attention_rows.hip, attention_rows_f32.hip); last, as in
+  // front of scale_log2 it cost the ragged step of 64 sequences 0.4%.
+  bool rows;
 };
 
 // Keys of token t (positions table in ragged mode); at least 1 (a position of
