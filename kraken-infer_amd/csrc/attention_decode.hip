@@ -1098,13 +1098,10 @@ SplitPlan plan_splits(const AttentionArgs& a, int cu_count) {
     }
   }
   if (rows) {
-    // The partials stay within the array that the allocation-free entry has, or
-    // within a smaller limit of the caller's.
-    const uint64_t limit = a.partial_limit < kNoAllocScratchBytes ? a.partial_limit
-                                                                  : kNoAllocScratchBytes;
+    // The partials stay within the array that the allocation-free entry has.
     const uint64_t per_split =
       (uint64_t)a.tokens * a.heads * (a.head_dim + 2u) * sizeof(float);
-    const uint64_t most = std::max<uint64_t>(1, limit / per_split);
+    const uint64_t most = std::max<uint64_t>(1, kNoAllocScratchBytes / per_split);
     kps = std::max(kps, most > 1 ? (max_keys + most - 1) / most : max_keys);
   }
   uint64_t splits = (max_keys + kps - 1) / kps;

@@ -188,27 +188,22 @@ int matmul_check(kraken_hip_context* ctx, int format, const kraken_buffer& weigh
 }
 
 // Whether a product of more than 8 tokens runs as kquant_mm.hip's two launches:
-// the faster form for `rows` (the largest matrix of a group), no form forced
-// through KRAKEN_KQUANT_GEMM, and a workspace that holds its packed inputs or
-// can grow to (not while the stream is captured, where an allocation would end
-// the capture; the other forms of a Q4_K product need no workspace).
-bool takes_mm(kraken_hip_context* ctx, int format, size_t rows, size_t cols, size_t tokens) {
-  if (!kquant_mm_supported(format, rows, cols, tokens) ||
-      std::getenv("KRAKEN_KQUANT_GEMM") != nullptr) {
-    return false;
-  }
-  return kquant_mm_workspace_bytes(cols, tokens) <= ctx->workspace_bytes || workspace_can_grow(ctx);
+// the faster form for `rows` (the largest matrix of a group) and no form forced
+// through KRAKEN_KQUANT_GEMM.
+bool takes_mm(int format, size_t rows, size_t cols, size_t tokens) {
+  return kquant_mm_supported(format, rows, cols, tokens) &&
+         std::getenv("KRAKEN_KQUANT_GEMM") == nullptr;
 }
 
 // launch_kquant_mm or launch_kquant_matmul for one matrix, with the workspace.
 int run_matmul(kraken_hip_context* ctx, int format, const std::string& p, const void* weight,
                size_t rows, size_t cols, size_t tokens, const float* input, const float* up,
                const float* residual, float* output) {
-  const bool mm = takes_mm(ctx, format, rows, cols, tokens);
+  const bool mm = takes_mm(format, rows, cols, tokens);
+  KRAKEN_TRY(begin_launch(ctx));
   KRAKEN_TRY(ensure_workspace(
     ctx, mm ? kquant_mm_workspace_bytes(cols, tokens)
             : kquant_matmul_workspace_bytes(format, rows, cols, tokens, up != nullptr)));
-  KRAKEN_TRY(begin_launch(ctx));
   const hipError_t e =
     mm ? launch_kquant_mm(format, 1, &weight, &rows, cols, tokens, input, up, residual, &output,
                           ctx->workspace, ctx->workspace_bytes, ctx->stream)
@@ -631,11 +626,11 @@ KRAKEN_API int kraken_hip_kquant_matmul_multi_f32(kraken_hip_context* ctx, size_
   }
   const char* group = std::getenv("KRAKEN_KQUANT_GROUP");
   if (same_format && (group == nullptr || std::strcmp(group, "off") != 0)) {
-    const bool mm = takes_mm(ctx, formats[0], *std::max_element(rows, rows + count), cols, tokens);
+    const bool mm = takes_mm(formats[0], *std::max_element(rows, rows + count), cols, tokens);
+    KRAKEN_TRY(begin_launch(ctx));
     if (mm) {
       KRAKEN_TRY(ensure_workspace(ctx, kquant_mm_workspace_bytes(cols, tokens)));
     }
-    KRAKEN_TRY(begin_launch(ctx));
     const float* x = static_cast<const float*>(input.data);
     const hipError_t e =
       mm ? launch_kquant_mm(formats[0], count, w, rows, cols, tokens, x, nullptr, nullptr, out,

@@ -103,23 +103,17 @@ int attention_entry(kraken_hip_context* ctx, const char* what, bool kv_f16,
 
   // An f16 query feeds the flash kernel as it is; the decode kernels read f32,
   // so that path widens it (exactly) into the workspace past the split partials.
+  size_t need = use_flash ? attention_flash_workspace_bytes(a, ctx->cu_count)
+                          : attention_decode_workspace_bytes(a, ctx->cu_count);
   size_t query_offset = 0;
-  auto needed = [&]() {
-    const size_t partials = use_flash ? attention_flash_workspace_bytes(a, ctx->cu_count)
-                                      : attention_decode_workspace_bytes(a, ctx->cu_count);
-    query_offset = query_f16 && !use_flash ? (partials + 255u) & ~size_t{255} : 0;
-    return query_f16 && !use_flash ? query_offset + query_values * sizeof(float) : partials;
-  };
-  size_t need = needed();
-  if (!no_alloc && need > ctx->workspace_bytes && !workspace_can_grow(ctx)) {
-    // Fewer key splits where that fits the workspace as it is.
-    const size_t query_bytes = query_f16 ? query_values * sizeof(float) + 255u : size_t{0};
-    a.partial_limit = ctx->workspace_bytes > query_bytes ? ctx->workspace_bytes - query_bytes : 0;
-    need = needed();
-  }
-  if (query_f16 && use_flash) {
-    a.query = nullptr;
-    a.query_f16 = query.data;
+  if (query_f16) {
+    if (use_flash) {
+      a.query = nullptr;
+      a.query_f16 = query.data;
+    } else {
+      query_offset = (need + 255u) & ~size_t{255};
+      need = query_offset + query_values * sizeof(float);
+    }
   }
   if (no_alloc && need > kNoAllocScratchBytes) {
     return invalid(w() + " needs " + std::to_string(need) +

@@ -90,7 +90,15 @@ int ensure_workspace(kraken_hip_context* ctx, size_t bytes) {
     rounded = 2 * ctx->workspace_bytes;
   }
   void* fresh = nullptr;
-  const hipError_t e = hipMalloc(&fresh, rounded);
+  // Relaxed for this thread meanwhile: while any stream is captured in the other
+  // modes an allocation fails and ends the capture.  It is no part of the graph,
+  // whose nodes only hold its address.
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  hipError_t e = hipThreadExchangeStreamCaptureMode(&mode);
+  if (e == hipSuccess) {
+    e = hipMalloc(&fresh, rounded);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
   if (e != hipSuccess) {
     return internal("HIP workspace allocation failed: " + hip_message(e));
   }
@@ -102,13 +110,6 @@ int ensure_workspace(kraken_hip_context* ctx, size_t bytes) {
   ctx->workspace = fresh;
   ctx->workspace_bytes = rounded;
   return KRAKEN_OK;
-}
-
-bool workspace_can_grow(const kraken_hip_context* ctx) {
-  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  return ctx->validation_only ||
-         (hipStreamIsCapturing(ctx->stream, &capture) == hipSuccess &&
-          capture == hipStreamCaptureStatusNone);
 }
 
 int check_u32(size_t value, const char* name) {

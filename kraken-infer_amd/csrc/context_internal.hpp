@@ -71,10 +71,6 @@ int finish_launch(kraken_hip_context* ctx, const char* a, const char* b, const c
 // address and nothing waits.  Returns KRAKEN_OK or an error status.
 int ensure_workspace(kraken_hip_context* ctx, size_t bytes);
 
-// Whether ensure_workspace may allocate now: not while the context's stream is
-// captured, where an allocation would end the capture.
-bool workspace_can_grow(const kraken_hip_context* ctx);
-
 // Size of the static per-device scratch array of the allocation-free entry
 // point, and the lookup of its device address on `device` (which must be the
 // current device); the address is resolved once per device and cached.
@@ -176,8 +172,6 @@ struct AttentionArgs {
   const uint32_t* seq_positions = nullptr;
   uint64_t pool_elems = 0;
   uint32_t max_position = 0;
-  // Most bytes of split partials that the several-token decode kernel may plan for.
-  size_t partial_limit = SIZE_MAX;
 };
 
 // Bytes of workspace the split-K decode path needs for these arguments.

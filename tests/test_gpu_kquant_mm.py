@@ -101,8 +101,7 @@ def test_group_equals_single(hip_ctx, ops, fmt):
 @pytest.mark.gpu
 def test_capture_without_a_grown_workspace():
     """A product that is captured before its context's workspace holds the packed
-    inputs takes a form that needs none (Q4_K), as an allocation would end the
-    capture; replays equal the eager result to rounding."""
+    inputs: the workspace grows, and replays have the eager result's bits."""
     import torch
 
     cols, rows, tokens = 1024, 2048, 1024
@@ -129,8 +128,7 @@ def test_capture_without_a_grown_workspace():
         ctx.matmul_q4_k_f32_device(wt, rows, cols, tokens, xt, out)
     torch.cuda.synchronize()
     for g in got:
-        assert torch.equal(g, got[0])
-        assert (g - out).abs().max() <= TOL * np.sqrt(cols) * out.abs().mean()
+        assert torch.equal(g, out)
     del graph
     ctx.commit_graph()
     ctx.close()
