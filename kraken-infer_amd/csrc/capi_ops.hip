@@ -102,18 +102,18 @@ int attention_entry(kraken_hip_context* ctx, const char* what, bool kv_f16,
                          (choice == FlashChoice::force_on || tokens >= 64u);
 
   // An f16 query feeds the flash kernel as it is; the decode kernels read f32,
-  // so that path widens it (exactly) into the workspace past the split partials.
+  // so that path widens it (exactly) into the workspace past the split partials
+  // (the plan must not see the f16 values' alignment: the kernels get the copy's).
+  if (query_f16) {
+    a.query = nullptr;
+    a.query_f16 = use_flash ? query.data : nullptr;
+  }
   size_t need = use_flash ? attention_flash_workspace_bytes(a, ctx->cu_count)
                           : attention_decode_workspace_bytes(a, ctx->cu_count);
   size_t query_offset = 0;
-  if (query_f16) {
-    if (use_flash) {
-      a.query = nullptr;
-      a.query_f16 = query.data;
-    } else {
-      query_offset = (need + 255u) & ~size_t{255};
-      need = query_offset + query_values * sizeof(float);
-    }
+  if (query_f16 && !use_flash) {
+    query_offset = (need + 255u) & ~size_t{255};
+    need = query_offset + query_values * sizeof(float);
   }
   if (no_alloc && need > kNoAllocScratchBytes) {
     return invalid(w() + " needs " + std::to_string(need) +

@@ -113,6 +113,34 @@ def test_rows_later_tokens_values_do_not_leak(hip_ctx, monkeypatch, bad):
     np.testing.assert_allclose(got[finite], one[finite], rtol=0, atol=8e-6)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens,start,heads,kv_heads", [
+    (40, 3000, 32, 8),   # the several-token kernel's splits, where one token's are one
+    (5, 9000, 8, 2),
+    (1, 4096, 8, 2),     # one token, split keys
+])
+@pytest.mark.parametrize("shift", [0, 1, 4])
+def test_f16_query_at_any_alignment(hip_ctx, tokens, start, heads, kv_heads, shift):
+    """An f16 query is widened into the workspace before these kernels read it, so
+    its own alignment changes nothing: the f32 entry's bits."""
+    torch = pytest.importorskip("torch")
+    print(f"rows f16 query tokens={tokens} heads={heads}/{kv_heads} shift={shift}", flush=True)
+    cap = start + tokens
+    q, k, v = inputs(11, tokens, start, cap, heads, kv_heads)
+    q = q.astype(np.float16)
+    want = kh.NumpyOps(hip_ctx).attention_batched(q.astype(np.float32), k, v, 0, start, tokens,
+                                                  cap, heads, kv_heads, D)
+    held = torch.zeros(q.size + 8, dtype=torch.float16, device="cuda")
+    view = held[shift:shift + q.size]
+    view.copy_(torch.from_numpy(q))
+    torch.cuda.synchronize()
+    kb, vb = hip_ctx.buffer(k), hip_ctx.buffer(v)
+    out = hip_ctx.buffer(byte_size=4 * q.size)
+    hip_ctx.attention_f16q_batched_f16_kv(view, kb, vb, 0, start, tokens, cap, heads, kv_heads, D,
+                                          out)
+    np.testing.assert_array_equal(out.download(q.size).view(np.uint32), want.view(np.uint32))
+
+
 @pytest.mark.parametrize("check", ["test_m0_has_no_other_user",
                                    "test_no_scc_value_lives_across_the_m0_add",
                                    "test_m0_write_never_directly_precedes_an_lds_dma_load"])
