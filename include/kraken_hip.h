@@ -706,7 +706,8 @@ KRAKEN_API int kraken_hip_kquant_top1_fused_f32(kraken_hip_context* context, uin
  * the largest of values[size]; NaN never wins, -inf can; all-NaN gives size.
  * argmax_prob_f32_i32 (mps_backend.hpp:387-390): also probability_output[0]
  * = 1 / sum_i exp(values[i] - max), or 0 when that sum is not positive.
- * Inputs above 16384 values use context workspace (12 bytes per 4096). */
+ * Inputs above 16384 values use context workspace: 12 bytes per 1024 values up
+ * to 262144 values, per 4096 above. */
 KRAKEN_API int kraken_hip_argmax_f32_i32(kraken_hip_context* context, kraken_buffer values,
                                          size_t size, kraken_buffer output);
 KRAKEN_API int kraken_hip_argmax_prob_f32_i32(kraken_hip_context* context, kraken_buffer values,

@@ -1895,8 +1895,12 @@ __global__ __launch_bounds__(256) void argmax_final_kernel(const float* values, 
 
 constexpr uint64_t kArgmaxSingleMax = 16384;  // one workgroup up to this size
 // Values per thread of a phase-1 workgroup: 16, or 4 where that gives at most the
-// 256 candidates that phase 2 takes in one pass and the workspace holds them.
+// 256 candidates that phase 2 takes in one pass.
 constexpr uint64_t kArgmaxPer = 16, kArgmaxPerSmall = 4;
+
+uint64_t argmax_per(uint64_t size) {
+  return size <= 256u * 256u * kArgmaxPerSmall ? kArgmaxPerSmall : kArgmaxPer;
+}
 
 template <int F>
 hipError_t launch_gemv_f(const GemvArgs& base, hipStream_t stream) {
@@ -2333,8 +2337,8 @@ size_t argmax_workspace_bytes(size_t size) {
   if (size <= kArgmaxSingleMax) {
     return 0;
   }
-  const size_t groups = (size + 256u * kArgmaxPer - 1) / (256u * kArgmaxPer);
-  return groups * sizeof(ArgCand);
+  const size_t span = 256u * argmax_per(size);
+  return (size + span - 1) / span * sizeof(ArgCand);
 }
 
 hipError_t launch_argmax(const float* values, size_t size, int32_t* token_out,
@@ -2346,16 +2350,13 @@ hipError_t launch_argmax(const float* values, size_t size, int32_t* token_out,
                                                token_out, probability_out);
     return hipGetLastError();
   }
-  size_t groups = (size + 256u * kArgmaxPerSmall - 1) / (256u * kArgmaxPerSmall);
-  const bool small = groups <= 256u && workspace_bytes >= groups * sizeof(ArgCand);
-  if (!small) {
-    groups = (size + 256u * kArgmaxPer - 1) / (256u * kArgmaxPer);
-  }
-  if (workspace == nullptr || workspace_bytes < groups * sizeof(ArgCand)) {
+  const size_t need = argmax_workspace_bytes(size);
+  if (workspace == nullptr || workspace_bytes < need) {
     return hipErrorInvalidValue;
   }
+  const size_t groups = need / sizeof(ArgCand);
   ArgCand* cands = static_cast<ArgCand*>(workspace);
-  if (small) {
+  if (argmax_per(size) == kArgmaxPerSmall) {
     argmax_partial_kernel<kArgmaxPerSmall>
       <<<dim3((uint32_t)groups), 256, 0, stream>>>(values, size, with_sum, cands);
   } else {

@@ -4,6 +4,7 @@ probability within 1e-5 as test_gpu_kquant.py holds it (an f32 sum of exponentia
 import numpy as np
 import pytest
 
+import kquant_cases as kc
 import kraken_hip as kh
 import oracle
 
@@ -26,3 +27,25 @@ def test_argmax_span_edges(hip_ctx, size):
             assert abs(p - want) <= 1e-5 * want
         else:
             assert p == want == 0.0
+
+
+@pytest.mark.gpu
+def test_top1_does_not_depend_on_the_workspace():
+    """261700 logits and their candidates fit a workspace of 1 MiB with 4096 values
+    per candidate and not with 1024: the same probability, bit for bit, from a new
+    context and from one whose workspace has grown."""
+    rows, cols = 261700, 256
+    print(f"top1 rows={rows} by workspace", flush=True)
+    w = kc.random_weight_fast("q4_k", rows, cols, seed=5)
+    x = np.random.default_rng(5).standard_normal(cols).astype(np.float32) / 16
+    got = []
+    for grown in (False, True):
+        ctx = kh.Context()
+        ops = kh.NumpyOps(ctx)
+        if grown:
+            ops.kquant_matmul("q5_k", kc.random_weight_fast("q5_k", 64, 1024, 1), 64, 1024,
+                              np.ones(2048 * 1024, np.float32), 2048)
+        token, p = ops.kquant_top1("q4_k", w, rows, cols, x, probability=True)
+        got.append((token, np.float32(p).view(np.uint32)))
+        ctx.close()
+    assert got[0] == got[1]
