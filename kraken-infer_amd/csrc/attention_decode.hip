@@ -1030,29 +1030,38 @@ bool tuned_args(const AttentionArgs& a) {
   return (d == 256 || d == 128 || d == 64) && (g == 1 || g == 2 || g == 4 || g == 8);
 }
 
-// Whether the several-token kernel runs: a sequence's 2 or more tokens with
-// head_dim 256, an f16 cache and up to 4 query heads per KV head, where one
-// workgroup per token would read many K/V rows again.  Its own launch takes about
-// 2 us longer on a short context, so the line lies at the rows that the tokens
-// read together.  Measured, us per call with prologue and merge, one workgroup per
-// token / this kernel, 2 KV heads x 4 query heads:
-//   37 tokens after  1500: 27.5 / 19.6  (114k rows read together)
-//   16 tokens after  1500: 16.6 / 18.5  ( 49k)
-//   63 tokens after   200: 16.8 / 16.2  ( 33k)
-//    3 tokens after  6144: 17.4 / 16.7  ( 37k)
-//    2 tokens after  6144: 14.5 / 14.9  ( 25k)
-//   37 tokens after  6144: 59.7 / 25.8
-//   63 tokens after 16384:  175 / 50.3
-// (4 x 2: 16 tokens after 1500 20.2 / 18.4, 37 after 6144 123 / 25.9.)
+// Whether a several-token kernel runs: a sequence's 2 or more tokens with head_dim
+// 256, an f16 cache and up to 4 query heads per KV head, where one workgroup per
+// token would read many K/V rows again.  Its launch and merge take 2 to 4 us longer
+// on a short context, so the line lies at the rows that the tokens read together.
+// Measured, us per call as a graph node with its merge, one workgroup per token /
+// this kernel, 2 KV heads x 4 query heads:
+//   33 tokens after  1000: 15.8 / 15.3  ( 68k rows read together)
+//   48 tokens after  1000: 23.0 / 15.6  (101k)
+//   24 tokens after  2000: 17.6 / 17.8  ( 97k)
+//   16 tokens after  3000: 15.8 / 15.9  ( 97k)
+//    4 tokens after  4096: 13.1 / 13.2  ( 33k)
+//    5 tokens after  4096: 15.1 / 14.2  ( 41k)
+//    3 tokens after  6144: 13.8 / 13.2  ( 37k)
+//   33 tokens after  6144: 55.6 / 21.4
+//   63 tokens after 10000:  111 / 33.9
+// (4 x 2: 12 after 2000 17.1 / 14.5; 2 after 4096 12.0 / 12.6.)  A context of one
+// split (kSingleSplitKeys) has few row groups to spread unless 4 heads share them:
+// 8 x 1, 48 after 200 12.8 / 14.5 (95k), 63 after 200 14.2 / 13.2 (133k); 8 x 4, 48
+// after 200 15.6 / 14.4.
 // Over an f32 cache, head_dim 64 or 128, the line lies at the multiplications that
-// the tokens' own workgroups do (8 KV heads x 2, head_dim 128):
-//   512 tokens after    0: 73.7 / 21.9;  after 2048: 456 / 99.4
-//   100 tokens after    0:  9.0 /  9.3  (21M);  after 100: 14.2 / 12.8  (41M)
-//    16 tokens after  500: 10.6 / 11.7  (17M)
-//     8 tokens after 2048: 14.6 / 11.9  (34M)
-// (head_dim 64, 4 x 1: 64 tokens after 512 5.9 / 10.0 (9M), 256 after 512 16.6 /
-// 9.5.  At head_dim 256 the operands of two tiles and O do not fit the registers:
-// 512 tokens, 2 x 4 heads 79 / 156.)
+// the tokens' own workgroups do, higher on a short context, whose keys they read
+// from the caches (8 KV heads x 2, head_dim 128, unless noted):
+//   128 tokens after    0: 10.3 /  9.4  (32M);  512 after 0 67.1 / 22.1
+//   100 tokens after    0:  8.8 /  9.3  (19M)
+//    24 tokens after  500: 11.1 / 12.0  (24M);  32 after 500 11.3 / 11.4  (33M)
+//    24 tokens after 1000: 18.7 / 13.5  (48M)
+//     8 tokens after 2048: 15.2 / 12.0  (32M)
+//   8 x 1: 128 after 100 11.0 / 12.7 (28M); 16 after 2048 21.2 / 12.5 (32M)
+//   1 x 1: 400 after 100 9.7 / 11.8 (24M); 200 after 1000 12.8 / 12.1 (29M)
+//   head_dim 64, 4 x 1: 200 after 300 11.0 / 8.5 (24M); 64 after 1000 8.0 / 10.1 (16M)
+// (At head_dim 256 the operands of two tiles and O do not fit the registers: 512
+// tokens, 2 x 4 heads 79 / 156.)
 // KRAKEN_DECODE_KERNEL forces one of the other kernels.
 bool takes_rows(const AttentionArgs& a) {
   if (a.seq_positions != nullptr || a.tokens < 2 || !tuned_args(a) ||
@@ -1063,10 +1072,12 @@ bool takes_rows(const AttentionArgs& a) {
   const uint64_t keys = (uint64_t)a.start_position + a.tokens;
   const uint64_t rows = keys * a.tokens * a.kv_heads;
   if (!a.kv_f16) {
-    return a.head_dim < 256u && rows * a.head_dim * g >= (24ull << 20);
+    const uint64_t line = a.head_dim == 128u && keys < 768u ? 32ull << 20 : 24ull << 20;
+    return a.head_dim < 256u && rows * a.head_dim * g >= line;
   }
   return a.head_dim == (uint32_t)kMD && g != 8 &&
-         (rows >= 81920u || (keys >= 4096u && rows >= 32768u));
+         (rows >= (keys > kSingleSplitKeys || g == 4 ? 81920u : 122880u) ||
+          (keys >= 4096u && rows >= 36864u));
 }
 
 SplitPlan plan_splits(const AttentionArgs& a, int cu_count) {

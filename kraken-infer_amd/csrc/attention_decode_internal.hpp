@@ -113,6 +113,37 @@ hipError_t launch_decode_short(const DecodeParams& p, uint32_t group, dim3 grid,
 hipError_t launch_decode_short_prologue(const DecodeParams& p, const PrologueFold& f,
                                         uint32_t group, hipStream_t stream);
 
+// A several-token workgroup's unit (split and KV head) and its place among the row
+// groups of that unit.  Consecutive workgroups go to consecutive XCDs.  Units that
+// divide among the eight XCDs keep their groups to one, whose L2 serves a unit's K/V
+// rows after the first group (rows_grid gives the places without a division).
+// Otherwise each XCD takes a run of the list, groups fastest, so that none gets more
+// than one workgroup more than another: with a unit's groups on one XCD some got up
+// to twice the workgroups of others (24 tokens after 2000 keys, 6 groups of 42
+// units: 27.5 us, in runs 17.7).  Fewer units than XCDs alternate, as a run would
+// hold one unit's longest groups only.
+struct RowsPlace {
+  uint32_t unit, order;
+};
+__host__ __device__ __forceinline__ bool rows_by_xcd(uint32_t units, uint32_t groups) {
+  return units % 8u == 0u && groups < 65536u;  // groups: a grid's y
+}
+__device__ __forceinline__ RowsPlace place_rows(uint32_t units, uint32_t groups) {
+  if (rows_by_xcd(units, groups)) {
+    return RowsPlace{8u * blockIdx.z + blockIdx.x, blockIdx.y};
+  }
+  if (units < 8u) {
+    return RowsPlace{blockIdx.x % units, blockIdx.x / units};
+  }
+  const uint32_t per = gridDim.x / 8u, rest = gridDim.x % 8u;
+  const uint32_t xcd = blockIdx.x % 8u;
+  const uint32_t id = xcd * per + min(xcd, rest) + blockIdx.x / 8u;
+  return RowsPlace{id / groups, id % groups};
+}
+inline dim3 rows_grid(uint32_t units, uint32_t groups) {
+  return rows_by_xcd(units, groups) ? dim3(8u, groups, units / 8u) : dim3(units * groups);
+}
+
 // Launches the several-token kernel (attention_rows.hip) for head_dim 256, an f16
 // cache and G in {1, 2, 4}: kRowsPerGroup query rows per workgroup.
 constexpr uint32_t kRowsPerGroup = 16;

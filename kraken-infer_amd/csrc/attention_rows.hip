@@ -51,17 +51,11 @@ __global__ __launch_bounds__(64 * kWaves) void attention_rows_kernel(DecodeParam
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15;
   const int kq = lane >> 4;
-  // The row groups of one (split, KV head) are eight workgroups apart: on one
-  // XCD, whose L2 serves their K/V rows after the first of them.
   const uint32_t groups = (p.tokens + kTokens - 1u) / kTokens;
-  const uint32_t within = blockIdx.x % (8u * groups);
-  const uint32_t unit = blockIdx.x / (8u * groups) * 8u + within % 8u;
-  if (unit >= p.splits * p.kv_heads) {
-    return;
-  }
-  const uint32_t split = unit / p.kv_heads;
-  const uint32_t kvh = unit % p.kv_heads;
-  const uint32_t first_token = within / 8u * kTokens;
+  const RowsPlace at_grid = place_rows(p.splits * p.kv_heads, groups);
+  const uint32_t split = at_grid.unit / p.kv_heads;
+  const uint32_t kvh = at_grid.unit % p.kv_heads;
+  const uint32_t first_token = at_grid.order * kTokens;
   const uint32_t last_token = min(first_token + kTokens, p.tokens) - 1u;
   const uint32_t key_begin = split * p.keys_per_split;
   const uint32_t most_keys = p.start_position + last_token + 1u;
@@ -369,7 +363,7 @@ __global__ __launch_bounds__(64 * kWaves) void attention_rows_kernel(DecodeParam
 hipError_t launch_decode_rows(const DecodeParams& p, uint32_t group, hipStream_t stream) {
   const uint32_t tokens = kRowsPerGroup / group;
   const uint32_t groups = (p.tokens + tokens - 1u) / tokens;
-  const dim3 grid((p.splits * p.kv_heads + 7u) / 8u * 8u * groups);
+  const dim3 grid = rows_grid(p.splits * p.kv_heads, groups);
   switch (group) {
     case 1: attention_rows_kernel<1><<<grid, 64 * kWaves, 0, stream>>>(p); break;
     case 2: attention_rows_kernel<2><<<grid, 64 * kWaves, 0, stream>>>(p); break;

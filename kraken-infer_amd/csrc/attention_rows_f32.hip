@@ -4,7 +4,7 @@
 // head, every product in f32 on v_mfma_f32_16x16x4_f32.
 //
 // One workgroup per token read its whole K/V range for one token's heads: 512
-// tokens (16 / 8 heads of 128) read 1 GB through the caches in 66 us.  Here a
+// tokens (16 / 8 heads of 128) read 1 GB through the caches in 67 us.  Here a
 // workgroup owns 16 query rows (16 / G consecutive tokens x G heads), a KV head
 // and a key split; its four waves take the split's 16-key tiles w, w + 4, ...
 //  * S^T = K Q^T: the MFMA's k index kq of step 4 j + e stands for dim
@@ -15,10 +15,10 @@
 //    n % 4, so a lane's V operands are float4s too, 256 consecutive bytes per key.
 //  * No operand goes through LDS; the next tile's loads are in flight while a tile
 //    computes (range-checked buffer loads: rows past the split read zeros).
-// A 16 x 16 tile is 4 D / 4 = D MFMAs of 32 cycles in all; what bounds the 512-token
-// chunk is that rate (1.1 GFLOP, 7 us at the card's f32 matrix peak) and the
-// causal imbalance, so a heavy row group and a light one share a CU: 73.7 -> 22.7 us
-// as a graph node, 165 -> 41.4 us after 500 tokens.
+// A 16 x 16 tile is D / 4 MFMAs for K Q^T and D / 4 for P V, of 32 cycles each; what
+// bounds the 512-token chunk is that rate (1.1 GFLOP, 7 us at the card's f32 matrix
+// peak) and the causal imbalance, so a heavy row group and a light one share a CU:
+// 67.1 -> 22.1 us as a node of a graph, 168 -> 41.9 us after 500 tokens.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -54,19 +54,14 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attention_rows_f32_kernel(Deco
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15;
   const int kq = lane >> 4;
-  // As attention_rows.hip; the row groups run from the last to the middle, then
-  // from the first: the two workgroups of a CU (half the grid apart) add up to
-  // about the same number of keys.
+  // The row groups run from the last to the middle, then from the first: the two
+  // workgroups of a CU (half the grid apart) add up to about the same number of keys.
   const uint32_t groups = (p.tokens + kTokens - 1u) / kTokens;
-  const uint32_t within = blockIdx.x % (8u * groups);
-  const uint32_t unit = blockIdx.x / (8u * groups) * 8u + within % 8u;
-  if (unit >= p.splits * p.kv_heads) {
-    return;
-  }
-  const uint32_t order = within / 8u, half = groups / 2u;
+  const RowsPlace at_grid = place_rows(p.splits * p.kv_heads, groups);
+  const uint32_t order = at_grid.order, half = groups / 2u;
   const uint32_t group = order < groups - half ? groups - 1u - order : order - (groups - half);
-  const uint32_t split = unit / p.kv_heads;
-  const uint32_t kvh = unit % p.kv_heads;
+  const uint32_t split = at_grid.unit / p.kv_heads;
+  const uint32_t kvh = at_grid.unit % p.kv_heads;
   const uint32_t first_token = group * kTokens;
   const uint32_t last_token = min(first_token + kTokens, p.tokens) - 1u;
   const uint32_t key_begin = split * p.keys_per_split;
@@ -342,7 +337,7 @@ hipError_t launch_decode_rows_f32(const DecodeParams& p, uint32_t head_dim, uint
                                   hipStream_t stream) {
   const uint32_t tokens = kRowsPerGroup / group;
   const uint32_t groups = (p.tokens + tokens - 1u) / tokens;
-  const dim3 grid((p.splits * p.kv_heads + 7u) / 8u * 8u * groups);
+  const dim3 grid = rows_grid(p.splits * p.kv_heads, groups);
   switch (head_dim) {
     case 64: return launch_dim<64>(p, group, grid, stream);
     case 128: return launch_dim<128>(p, group, grid, stream);

@@ -36,6 +36,8 @@ def inputs(seed, tokens, start, cap, heads, kv_heads, layers=1, scale=1.0):
     (33, 4100, 8, 4, 1.0),     # G = 2
     (63, 1300, 8, 2, 8.0),     # the most tokens before flash
     (63, 700, 4, 2, 1.0),      # the shortest context at two KV heads
+    (25, 2100, 12, 3, 1.0),    # a grid that is no multiple of the eight XCDs
+    (11, 5000, 2, 1, 1.0),     # one KV head
 ])
 def test_rows_against_oracle(hip_ctx, monkeypatch, tokens, start, heads, kv_heads, scale):
     print(f"rows tokens={tokens} start={start} heads={heads}/{kv_heads}", flush=True)

@@ -25,7 +25,10 @@ def inputs(seed, tokens, cap, heads, kv_heads, d, layers=1):
     (512, 0, 16, 8, 128),     # a prefill chunk: one split, 64 row groups
     (129, 900, 8, 8, 128),    # G = 1, the last group holds one token
     (37, 2100, 8, 2, 128),    # G = 4, splits
-    (100, 0, 16, 8, 128), (101, 30, 16, 8, 128),  # either side of the rule
+    (100, 0, 16, 8, 128), (101, 30, 16, 8, 128),
+    (127, 0, 16, 8, 128), (128, 0, 16, 8, 128),   # either side of the rule
+    (31, 737, 16, 8, 128), (32, 735, 16, 8, 128),  # and of its line for short contexts
+    (90, 700, 8, 1, 128),     # G = 8, fewer splits than XCDs
     (21, 3000, 16, 2, 128),   # G = 8, two tokens per group, the last one alone
     (2, 70000, 4, 2, 128),    # a quarter of one group over many splits
     (175, 800, 4, 4, 64), (97, 601, 8, 1, 64),
