@@ -20,6 +20,74 @@ namespace {
 
 constexpr int kWaves = 4;
 
+// A wave per token and head.
+__global__ __launch_bounds__(256) void attention_prologue_head_kernel(PrologueArgs a) {
+  const int lane = threadIdx.x & 63;
+  const uint32_t slots = a.heads + 2u * a.kv_heads;
+  const size_t item = (size_t)blockIdx.x * kWaves + (threadIdx.x >> 6);
+  if (item >= (size_t)a.tokens * slots) {
+    return;  // whole wave
+  }
+  const uint32_t t = (uint32_t)(item / slots);
+  const uint32_t slot = (uint32_t)(item % slots);
+  const uint32_t d_head = a.head_dim;
+  const size_t kv_dim = (size_t)a.kv_heads * d_head;
+
+  if (slot >= a.heads + a.kv_heads) {  // value head: f32 -> f16 append
+    const uint32_t kh = slot - a.heads - a.kv_heads;
+    const float* src = a.value + (size_t)t * kv_dim + (size_t)kh * d_head;
+    half_t* dst = a.value_cache + a.cache_offset + (size_t)t * kv_dim + (size_t)kh * d_head;
+    for (uint32_t d = lane; d < d_head; d += 64) {
+      dst[d] = static_cast<half_t>(src[d]);
+    }
+    return;
+  }
+
+  const bool is_q = slot < a.heads;
+  const uint32_t head = is_q ? slot : slot - a.heads;
+  const float* src = is_q ? a.q_gate + ((size_t)t * a.heads + head) * 2u * d_head
+                          : a.key + (size_t)t * kv_dim + (size_t)head * d_head;
+  const float* weight = is_q ? a.q_norm : a.k_norm;
+  const RopeArgs rope{a.positions, a.mrope_start, a.tokens, a.n_dims, a.s0, a.s1, a.s2, a.s3,
+                      a.theta};
+  float v[4], w[4], g[4];
+  load_head(src, weight, d_head, lane, v, w);
+  // The gate half of a q_gate head is copied out; its loads go out with the rest.
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t d = lane + 64u * i;
+    g[i] = is_q && d < d_head ? src[d_head + d] : 0.0f;
+  }
+  int32_t pos[4];
+  rope_positions(rope, t, pos);
+  double sn[4], cs[4];
+  rope_angles(rope, pos, lane, sn, cs);
+  float r[4];
+  norm_rope(v, w, d_head, a.eps, a.n_dims, sn, cs, lane, r);
+
+  if (is_q) {
+    float* q_out = a.query_out + ((size_t)t * a.heads + head) * d_head;
+    float* g_out = a.gate_out + ((size_t)t * a.heads + head) * d_head;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t d = lane + 64u * i;
+      if (d < d_head) {
+        q_out[d] = r[i];
+        g_out[d] = g[i];
+      }
+    }
+  } else {
+    half_t* dst = a.key_cache + a.cache_offset + (size_t)t * kv_dim + (size_t)head * d_head;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t d = lane + 64u * i;
+      if (d < d_head) {
+        dst[d] = static_cast<half_t>(r[i]);
+      }
+    }
+  }
+}
+
 // A wave takes H consecutive heads of one token (query, then key, then value
 // heads); the token's rotation angles (a pow and a sincos in double per pair) are
 // computed once for them.
@@ -132,16 +200,21 @@ hipError_t launch_attention_prologue(const PrologueArgs& a, hipStream_t stream) 
   if (a.tokens == 0) {
     return hipSuccess;
   }
-  // Heads per wave: one where few waves run, whose latency then counts (each more
-  // costs 0.7 us: 1 token 12.1 / 12.8 / 13.5 us with 1 / 2 / 3, the attention
-  // included); from 256 tokens on up to four, so that the angles are formed less
-  // often.  Three where that divides a token's heads over one workgroup's waves.
-  // Attention core of 1024 tokens after 500, 1 / 3 / 4 heads per wave: 8 + 2 + 2
-  // heads 42.4 / 39.7 / 38.3 us (512 tokens 33.1 / 29.7 / 32.2), 8 + 4 + 4 heads
-  // 53.3 / 50.4 / 46.6, 16 + 4 + 4 heads 66.4 / 60.2 / 58.0.
+  // Heads per wave: one where few waves run, whose latency then counts; from 256
+  // tokens and 4096 heads on (3072 where more than 64 elements rotate) up to four, so
+  // that the angles are formed less often.  Three where that divides a token's heads
+  // over one workgroup's waves.  Measured, us, one / several heads per wave (q + k + v
+  // heads of 256, n_dims 64):
+  //   8 + 2 + 2  300 tokens 6.3 / 6.6   400 7.5 / 6.9   1024 14.6 / 11.3
+  //   4 + 2 + 2  300 tokens 5.5 / 5.6   512 6.5 / 6.7    700  8.6 /  8.1
+  //   4 + 1 + 1  512 tokens 5.5 / 5.8   700 7.1 / 6.7
+  //   1 + 1 + 1  512 tokens 4.3 / 5.3  1024 5.4 / 5.7   2048  8.0 /  6.9
+  //   8 + 4 + 4  128 tokens 4.5 / 6.2   256 6.8 / 6.7   1024 18.2 / 12.7
+  //   8 + 2 + 2, n_dims 256  128 tokens 8.8 / 8.7  256 11.7 / 9.1
   const size_t slots = a.heads + 2u * (size_t)a.kv_heads;
-  if (a.tokens < 256u) {
-    launch_heads<1>(a, stream);
+  if (a.tokens < 256u || a.tokens * slots < (a.n_dims <= 64u ? 4096u : 3072u)) {
+    const size_t blocks = (a.tokens * slots + kWaves - 1) / kWaves;
+    attention_prologue_head_kernel<<<dim3((uint32_t)blocks), 256, 0, stream>>>(a);
   } else if (slots <= 12u) {
     launch_heads<3>(a, stream);
   } else {

@@ -71,6 +71,37 @@ __device__ __forceinline__ void rope_angles(const RopeArgs& a, const int32_t pos
   }
 }
 
+// The rotation of elements lane + 64 i, i < kRegs, of a normed head; n_dims <= 64
+// kRegs.  Pairs (p, p + n_dims / 2), p < n_dims / 2: each lane fetches the partner of
+// each of its elements from the lane and register that hold it.
+template <int kRegs>
+__device__ __forceinline__ void rotate_head(const float v[4], uint32_t n_dims, const double sn[4],
+                                            const double cs[4], int lane, float r[4]) {
+  const uint32_t half_dims = n_dims / 2u;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    r[i] = v[i];
+    if (i >= kRegs) {
+      continue;
+    }
+    const uint32_t e = lane + 64u * i;
+    const uint32_t p = e < half_dims ? e + half_dims : (e < n_dims ? e - half_dims : e);
+    const int src_lane = (int)(p & 63u);
+    const uint32_t src_reg = p >> 6;
+    float partner = 0.0f;
+#pragma unroll
+    for (int j = 0; j < kRegs; ++j) {
+      const float x = __shfl(v[j], src_lane, 64);
+      partner = src_reg == (uint32_t)j ? x : partner;
+    }
+    if (e < n_dims) {
+      const double x0 = e < half_dims ? v[i] : partner;
+      const double x1 = e < half_dims ? partner : v[i];
+      r[i] = e < half_dims ? (float)(x0 * cs[i] - x1 * sn[i]) : (float)(x1 * cs[i] + x0 * sn[i]);
+    }
+  }
+}
+
 // r = MRoPE(v * rsqrt(mean(v^2) + eps) * w): elements past d_head are 0, those
 // in [n_dims, d_head) only normalised.
 __device__ __forceinline__ void norm_rope(const float v_in[4], const float w[4], uint32_t d_head,
@@ -90,32 +121,16 @@ __device__ __forceinline__ void norm_rope(const float v_in[4], const float w[4],
     const uint32_t d = lane + 64u * i;
     v[i] = d < d_head ? v[i] * scale * w[i] : 0.0f;
   }
-
-  // Pairs (p, p + n_dims / 2), p < n_dims / 2.  Each lane fetches the partner
-  // of each of its elements from the lane and register that hold it.
-  const uint32_t half_dims = n_dims / 2u;
+  // One exchange for a rotation within 64 elements; the sixteen of any other in one
+  // block (a branch around each made every exchange wait for the one before: a
+  // head of 256 rotated elements 7.1 -> 7.6 us for 17 tokens).
+  if (n_dims <= 64u) {
+    rotate_head<1>(v, n_dims, sn, cs, lane, r);
+  } else {
+    rotate_head<4>(v, n_dims, sn, cs, lane, r);
+  }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const uint32_t e = lane + 64u * i;
-    r[i] = v[i];
-    if (64u * i < n_dims) {  // wave-uniform: the rotation reaches these elements
-      const uint32_t p = e < half_dims ? e + half_dims : (e < n_dims ? e - half_dims : e);
-      const int src_lane = (int)(p & 63u);
-      const uint32_t src_reg = p >> 6;
-      float partner = 0.0f;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (64u * j < n_dims) {  // partners lie below n_dims
-          const float x = __shfl(v[j], src_lane, 64);
-          partner = src_reg == (uint32_t)j ? x : partner;
-        }
-      }
-      if (e < n_dims) {
-        const double x0 = e < half_dims ? v[i] : partner;
-        const double x1 = e < half_dims ? partner : v[i];
-        r[i] = e < half_dims ? (float)(x0 * cs[i] - x1 * sn[i]) : (float)(x1 * cs[i] + x0 * sn[i]);
-      }
-    }
     // The f32 result kept as such: a caller that rounds it to fp16 (the K
     // append) must not get the norm's last multiply and that rounding fused
     // into one v_fma_mix, which the separate qk_norm / mrope / copy ops (each
