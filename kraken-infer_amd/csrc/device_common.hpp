@@ -256,4 +256,41 @@ __device__ __forceinline__ void store_through(float* at, float v) {
   __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// A lane's sums of a matrix product into c [tokens][n]: v[i] for row `row` and token
+// token(i), or residual + v[i] (the residual may be c itself).  The residuals are all
+// requested before the first is used: a load in front of each store made the N of
+// them wait for memory in turn (K-quant Q6_K 3584 x 1024, 512 tokens: 38.4 us, 21.3
+// so, against 20.5 without a residual).
+template <int N, class Token>
+__device__ __forceinline__ void store_sums(float* c, const float* residual, uint32_t n,
+                                           uint32_t row, uint32_t tokens, Token token,
+                                           const float (&v)[N]) {
+  if (row >= n) {
+    return;
+  }
+  float r[N];
+  if (residual != nullptr) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      // Past the last token: the lane's element of the last one, not used.
+      r[i] = residual[(uint64_t)min(token(i), tokens - 1u) * n + row];
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      r[i] += v[i];
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      r[i] = v[i];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    if (token(i) < tokens) {
+      store_through(&c[(uint64_t)token(i) * n + row], r[i]);
+    }
+  }
+}
+
 }  // namespace kraken

@@ -1325,14 +1325,14 @@ __global__ __launch_bounds__(256) void gemm_f16_nt_kernel(const half_t* x, const
 #pragma unroll
     for (int j = 0; j < JB; ++j) {
       const uint32_t col = n0 + (TN / 2) * wn + 32u * j + (uint32_t)frow;
+      float v[16];
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const uint32_t row = m0 + (TM / 2) * wm + 32u * i + 8u * (e / 4) + 4u * fk + (e % 4);
-        if (row < m && col < n) {
-          const uint64_t at = (uint64_t)row * n + col;
-          store_through(&c[at], residual != nullptr ? residual[at] + acc[i][j][e] : acc[i][j][e]);
-        }
+        v[e] = acc[i][j][e];
       }
+      store_sums(c, residual, n, col, m, [&](int e) {
+        return m0 + (TM / 2) * wm + 32u * i + 8u * (e / 4) + 4u * fk + (e % 4);
+      }, v);
     }
   }
 }
@@ -1493,14 +1493,14 @@ __global__ __launch_bounds__(256) void gemm_f16_pipe_kernel(const half_t* x, con
 #pragma unroll
     for (int j = 0; j < JB; ++j) {
       const uint32_t col = n0 + (TN / 2) * wn + 32u * j + (uint32_t)frow;
+      float v[16];
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const uint32_t row = m0 + (TM / 2) * wm + 32u * i + 8u * (e / 4) + 4u * fk + (e % 4);
-        if (row < m && col < n) {
-          const uint64_t at = (uint64_t)row * n + col;
-          store_through(&c[at], residual != nullptr ? residual[at] + acc[i][j][e] : acc[i][j][e]);
-        }
+        v[e] = acc[i][j][e];
       }
+      store_sums(c, residual, n, col, m, [&](int e) {
+        return m0 + (TM / 2) * wm + 32u * i + 8u * (e / 4) + 4u * fk + (e % 4);
+      }, v);
     }
   }
 }
@@ -1685,14 +1685,14 @@ __global__ __launch_bounds__(256) void gemm_kq_kernel(const float* x, const uint
 #pragma unroll
     for (int j = 0; j < JB; ++j) {
       const uint32_t col = n0 + (TN / 2) * wn + 32u * j + (uint32_t)frow;
+      float v[16];
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const uint32_t row = m0 + (TM / 2) * wm + 32u * i + 8u * (e / 4) + 4u * fk + (e % 4);
-        if (row < m && col < n) {
-          const uint64_t at = (uint64_t)row * n + col;
-          store_through(&c[at], residual != nullptr ? residual[at] + acc[i][j][e] : acc[i][j][e]);
-        }
+        v[e] = acc[i][j][e];
       }
+      store_sums(c, residual, n, col, m, [&](int e) {
+        return m0 + (TM / 2) * wm + 32u * i + 8u * (e / 4) + 4u * fk + (e % 4);
+      }, v);
     }
   }
 }

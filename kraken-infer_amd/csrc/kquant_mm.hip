@@ -285,41 +285,6 @@ __device__ __forceinline__ MmTile locate_tile(const MmArgs& a) {
   return MmTile{g, tile * kRows, id % a.token_tiles * kTokens};
 }
 
-// Output elements (row, token(i)), i < N, of a matrix with n rows: the sums, or
-// residual + sums.  The residuals are all requested before the first is used: a load
-// in front of each store made the N of them wait for memory in turn (Q6_K 3584 x
-// 1024, 512 tokens: twice the time of the product without a residual).
-template <int N, class Token>
-__device__ __forceinline__ void store_sums(const MmArgs& a, float* c, uint32_t n, uint32_t row,
-                                           Token token, const float (&v)[N]) {
-  if (row >= n) {
-    return;
-  }
-  float r[N];
-  if (a.residual != nullptr) {
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      // Past the last token: the lane's element of the last one, not used.
-      r[i] = a.residual[(uint64_t)min(token(i), a.tokens - 1u) * n + row];
-    }
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      r[i] += v[i];
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      r[i] = v[i];
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    if (token(i) < a.tokens) {
-      store_through(&c[(uint64_t)token(i) * n + row], r[i]);
-    }
-  }
-}
-
 // Few tokens, or few rows: the KW waves of a workgroup split the K blocks of one
 // tile of 32 RA rows x 32 TB tokens and add their sums through LDS in wave order.
 // No wave waits for another before that, and each has a whole stage of pieces
@@ -478,7 +443,7 @@ __global__ __launch_bounds__(64 * KW, 2) void kq_mm_kernel(MmArgs a) {
       v[i] += s_sum[k][reg][lane];
     }
   }
-  store_sums(a, a.c[g], n, n0 + 32u * (wave * kShare / (16u * TB)) + r32, [&](int i) {
+  store_sums(a.c[g], a.residual, n, n0 + 32u * (wave * kShare / (16u * TB)) + r32, a.tokens, [&](int i) {
     const uint32_t reg = wave * kShare + i;
     const uint32_t e = reg % 16u, t = reg / 16u % TB;
     return t0 + 32u * t + 8u * (e / 4u) + 4u * kh + (e % 4u);
@@ -635,7 +600,7 @@ void kq_mm_lds_kernel(MmArgs a) {
     for (int e = 0; e < 16; ++e) {
       v[e] = acc[t][e];
     }
-    store_sums(a, a.c[g], n, n0 + r32, [&](int e) {
+    store_sums(a.c[g], a.residual, n, n0 + r32, a.tokens, [&](int e) {
       return t0 + 32u * t + 8u * (e / 4) + 4u * kh + (e % 4);
     }, v);
   }
