@@ -609,57 +609,53 @@ void kq_mm_lds_kernel(MmArgs a) {
 // X [tokens][cols] f32 -> fp16 pieces [token group of 32][k / 16][lane][8]:
 // lane l holds token l % 32 and k = 16 s + 8 (l / 32) .. + 7; tokens past the
 // input are zero.  With up, X is silu(x) * up (silu_mul_f32_in_place's
-// arithmetic).  One wave per kPackSteps pieces.
-constexpr uint32_t kPackSteps = 4;
+// arithmetic).  One wave per piece: bound by latency, so that with four pieces per
+// wave the products took 0.4 to 0.8 us longer, and 2.0 to 2.4 us with up, whose
+// exponentials then form one chain (48 tokens x 1024, Q4_K 3584 rows: 6.9 -> 6.2
+// us, with up 9.0 -> 6.6).
 template <bool kSwiglu>
 __global__ __launch_bounds__(256) void kq_pack_x_kernel(const float* x, const float* up,
                                                         half_t* out, uint32_t tokens,
                                                         uint32_t cols, uint32_t pieces) {
 #pragma clang fp contract(off)
   const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t first = (blockIdx.x * 4u + (threadIdx.x >> 6)) * kPackSteps;
-  if (first >= pieces) {
+  const uint32_t piece = blockIdx.x * 4u + (threadIdx.x >> 6);
+  if (piece >= pieces) {
     return;
   }
-  const uint32_t per_group = cols / 16u;  // a multiple of 16: a wave stays in one group
-  const uint32_t token = first / per_group * 32u + (lane & 31u);
-  const uint32_t k = first % per_group * 16u + 8u * (lane >> 5);
-  float4 v[kPackSteps][2], u[kPackSteps][2];
+  const uint32_t per_group = cols / 16u;
+  const uint32_t token = piece / per_group * 32u + (lane & 31u);
+  const uint32_t k = piece % per_group * 16u + 8u * (lane >> 5);
+  float4 v[2], u[2];
 #pragma unroll
-  for (uint32_t s = 0; s < kPackSteps; ++s) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      v[s][i] = make_float4(0.f, 0.f, 0.f, 0.f);
-      u[s][i] = v[s][i];
-      if (token < tokens) {
-        const uint64_t at = ((uint64_t)token * cols + k + 16u * s + 4u * i) / 4u;
-        v[s][i] = reinterpret_cast<const float4*>(x)[at];
-        if constexpr (kSwiglu) {
-          u[s][i] = reinterpret_cast<const float4*>(up)[at];
-        }
+  for (int i = 0; i < 2; ++i) {
+    v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    u[i] = v[i];
+    if (token < tokens) {
+      const uint64_t at = ((uint64_t)token * cols + k + 4u * i) / 4u;
+      v[i] = reinterpret_cast<const float4*>(x)[at];
+      if constexpr (kSwiglu) {
+        u[i] = reinterpret_cast<const float4*>(up)[at];
       }
     }
   }
+  half8_t h;
 #pragma unroll
-  for (uint32_t s = 0; s < kPackSteps; ++s) {
-    half8_t h;
+  for (int i = 0; i < 2; ++i) {
+    const float f[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+    const float q[4] = {u[i].x, u[i].y, u[i].z, u[i].w};
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const float f[4] = {v[s][i].x, v[s][i].y, v[s][i].z, v[s][i].w};
-      const float q[4] = {u[s][i].x, u[s][i].y, u[s][i].z, u[s][i].w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float y = f[e];
-        if constexpr (kSwiglu) {
-          // The f32 product kept as such before its rounding to fp16.
-          y = (y / (1.0f + expf(-y))) * q[e];
-          asm("" : "+v"(y));
-        }
-        h[4 * i + e] = static_cast<half_t>(y);
+    for (int e = 0; e < 4; ++e) {
+      float y = f[e];
+      if constexpr (kSwiglu) {
+        // The f32 product kept as such before its rounding to fp16.
+        y = (y / (1.0f + expf(-y))) * q[e];
+        asm("" : "+v"(y));
       }
+      h[4 * i + e] = static_cast<half_t>(y);
     }
-    reinterpret_cast<half8_t*>(out)[(uint64_t)(first + s) * 64u + lane] = h;
   }
+  reinterpret_cast<half8_t*>(out)[(uint64_t)piece * 64u + lane] = h;
 }
 
 template <class S>
@@ -784,7 +780,7 @@ hipError_t launch_kquant_mm(int format, size_t count, const void* const* weights
   a.cols = (uint32_t)cols;
   const MmForm form = mm_form(format, most_rows, cols, tokens);
   const uint32_t pieces = (uint32_t)((tokens + 31u) / 32u * (cols / 16u));
-  const dim3 grid((pieces + 4u * kPackSteps - 1u) / (4u * kPackSteps));
+  const dim3 grid((pieces + 3u) / 4u);
   half_t* packed = static_cast<half_t*>(workspace);
   if (up != nullptr) {
     kq_pack_x_kernel<true><<<grid, 256, 0, stream>>>(input, up, packed, a.tokens, a.cols, pieces);
