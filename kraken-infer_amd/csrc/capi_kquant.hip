@@ -14,7 +14,6 @@
 // allocation of this library or of torch is.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <string>
@@ -188,18 +187,18 @@ int matmul_check(kraken_hip_context* ctx, int format, const kraken_buffer& weigh
 }
 
 // Whether a product of more than 8 tokens runs as kquant_mm.hip's two launches:
-// the faster form for `rows` (the largest matrix of a group) and no form forced
-// through KRAKEN_KQUANT_GEMM.
-bool takes_mm(int format, size_t rows, size_t cols, size_t tokens) {
-  return kquant_mm_supported(format, rows, cols, tokens) &&
-         std::getenv("KRAKEN_KQUANT_GEMM") == nullptr;
+// the faster form for these matrices and no form forced through
+// KRAKEN_KQUANT_GEMM.
+bool takes_mm(int format, size_t count, const size_t* rows, size_t cols, size_t tokens) {
+  return std::getenv("KRAKEN_KQUANT_GEMM") == nullptr &&
+         kquant_mm_supported(format, count, rows, cols, tokens);
 }
 
 // launch_kquant_mm or launch_kquant_matmul for one matrix, with the workspace.
 int run_matmul(kraken_hip_context* ctx, int format, const std::string& p, const void* weight,
                size_t rows, size_t cols, size_t tokens, const float* input, const float* up,
                const float* residual, float* output) {
-  const bool mm = takes_mm(format, rows, cols, tokens);
+  const bool mm = takes_mm(format, 1, &rows, cols, tokens);
   KRAKEN_TRY(begin_launch(ctx));
   KRAKEN_TRY(ensure_workspace(
     ctx, mm ? kquant_mm_workspace_bytes(cols, tokens)
@@ -626,7 +625,7 @@ KRAKEN_API int kraken_hip_kquant_matmul_multi_f32(kraken_hip_context* ctx, size_
   }
   const char* group = std::getenv("KRAKEN_KQUANT_GROUP");
   if (same_format && (group == nullptr || std::strcmp(group, "off") != 0)) {
-    const bool mm = takes_mm(formats[0], *std::max_element(rows, rows + count), cols, tokens);
+    const bool mm = takes_mm(formats[0], count, rows, cols, tokens);
     KRAKEN_TRY(begin_launch(ctx));
     if (mm) {
       KRAKEN_TRY(ensure_workspace(ctx, kquant_mm_workspace_bytes(cols, tokens)));

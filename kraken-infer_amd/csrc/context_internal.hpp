@@ -359,14 +359,18 @@ hipError_t launch_kquant_matmul(int format, const void* weight, size_t rows, siz
 // The two launches of kquant_mm.hip (input packing, then the product with the
 // weights decoded in registers): up to kKquantGroupMax matrices of one format
 // over the same input, with `up` as above; `residual` with one matrix only.
-// supported: whether this is the faster form for that many rows (of the group's
-// largest matrix).
-bool kquant_mm_supported(int format, size_t rows, size_t cols, size_t tokens);
+// supported: whether this is the faster form for these matrices (without up or
+// residual, so that a folded product has the bits of the separate operations).
+bool kquant_mm_supported(int format, size_t count, const size_t* rows, size_t cols,
+                         size_t tokens);
 size_t kquant_mm_workspace_bytes(size_t cols, size_t tokens);
 hipError_t launch_kquant_mm(int format, size_t count, const void* const* weights,
                             const size_t* rows, size_t cols, size_t tokens, const float* input,
                             const float* up, const float* residual, float* const* outputs,
                             void* workspace, size_t workspace_bytes, hipStream_t stream);
+// The estimated time in us of launch_kquant_matmul for these matrices, or of
+// launch_kquant_matmul_group where the format runs them as one launch.
+double kquant_matmul_us(int format, size_t count, const size_t* rows, size_t cols, size_t tokens);
 // Up to kKquantGroupMax matmuls of one format that share input, cols and
 // tokens (kquant.hip).  More than kKquantGemvMaxTokens tokens with the fused
 // GEMM form (weights decoded in the B tile) run as one launch whose grid holds

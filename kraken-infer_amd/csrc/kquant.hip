@@ -2177,6 +2177,39 @@ hipError_t launch_kquant_matmul_group(int format, size_t count, const void* cons
   return hipGetLastError();
 }
 
+double kquant_matmul_us(int format, size_t count, const size_t* rows, size_t cols,
+                        size_t tokens) {
+  // The passes, and per round of 256 workgroups the K steps (fitted as mm_us in
+  // kquant_mm.hip says).
+  const bool b_tile = format == 0;
+  const double step[3] = {0.58, 0.85, 1.05}, weight[3] = {0.0, 0.56, 0.72};
+  double us = 0.0;
+  uint64_t b_tiles = 0;
+  for (size_t i = 0; i < count; ++i) {
+    const uint64_t token_tiles = (tokens + 127) / 128;
+    const double outputs = 1e-6 * (double)rows[i] * (double)tokens;
+    const uint32_t splits = b_tile && count > 1 ? 1u : gemm_k_splits(rows[i], cols, tokens);
+    const double steps = (double)((cols / kGK + splits - 1) / splits);
+    if (b_tile) {
+      b_tiles += (rows[i] + 127) / 128 * token_tiles * splits;
+      us += 0.23 * outputs + (splits > 1 ? 1.13 + 1.79 * splits * outputs : 0.0);
+      if (i + 1 == count) {
+        us += 1.1 + (double)((b_tiles + 255) / 256) * (1.116 * steps + 2.43);
+      }
+      continue;
+    }
+    const GemmKernel kernel = gemm_f16_kernel_choice(rows[i], tokens, splits);
+    const int k = kernel == GemmKernel::pipe192 ? 1 : (kernel == GemmKernel::pipe256 ? 2 : 0);
+    const uint64_t tile_rows = 128u + 64u * k;
+    const uint64_t workgroups = (rows[i] + tile_rows - 1) / tile_rows * token_tiles * splits;
+    us += 5.1 + 1e-6 * weight[format] * (double)rows[i] * (double)cols +
+          0.89e-6 * (double)tokens * (double)cols + 0.48 * outputs +
+          (double)((workgroups + 255) / 256) * (steps * step[k] + 0.96 * (1.0 + 0.5 * k)) +
+          (splits > 1 ? 2.1 + 1.23 * splits * outputs : 0.0);
+  }
+  return us;
+}
+
 // Input groups of eight from which the first pass converts four per thread.
 constexpr uint64_t kWideConvertGroups = 262144;
 

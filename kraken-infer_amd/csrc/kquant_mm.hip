@@ -681,26 +681,28 @@ void launch_lds(MmArgs a, hipStream_t stream) {
   kq_mm_lds_kernel<F, RW><<<grid, LdsShape<RW>::kThreads, 0, stream>>>(a);
 }
 
-// The tile shapes, smallest first.
+// The tile shapes, smallest first.  Whether they or the older forms run: mm_us.
 enum class MmForm { two_pass, split_32x32, split_32x64, split_64x64, lds_64, lds_128, lds_256 };
 
 // The smallest tile whose workgroups do not exceed the chip's 256 CUs (about two
-// each for the 64 x 64 tile), counted for one matrix of `rows` rows so that a
-// matrix gets the same form, and the same bits, in a group and on its own.
-// Measured at 1024 columns, us per call with the packing launch, 32x32 / 32x64 /
-// 64x64 / 128x128 / 256x128 tiles:
-//   Q4_K 6144 rows   32 tokens   6.9 /  8.1 /  9.3 /    - /    -   (192 of 32x32)
-//                   128 tokens  10.8 / 11.2 / 10.3 / 16.6 / 20.6   (192 of 64x64)
-//                   256 tokens  16.2 / 14.9 / 14.4 / 17.0 / 20.8   (384 of 64x64)
-//                   384 tokens  21.7 / 20.1 / 19.6 / 17.5 / 21.4   (576 of 64x64)
-//                   768 tokens  36.9 / 31.3 / 28.1 / 26.3 / 23.0   (144 of 256x128)
-//                  1024 tokens  49.0 / 40.2 / 33.0 / 27.8 / 26.3
-//   Q4_K 3584 rows 1024 tokens  31.8 / 27.6 / 24.6 / 20.0 / 23.0   (112 of 256x128)
+// each for the 64 x 64 tile), counted for one matrix of `rows` rows (the largest of a
+// group: only matrices of that size get the same tiles, and the same bits, in a group
+// and on their own).  Measured at 1024 columns, us per call with the packing launch,
+// 32x32 / 32x64 / 64x64 / 128x128 / 256x128 tiles:
+//   Q4_K 6144 rows   32 tokens   7.1 /  8.2 /  9.3 / 15.6 / 19.6   (192 of 32x32)
+//                   128 tokens  10.8 / 10.8 /  9.9 / 16.0 / 20.2   (192 of 64x64)
+//                   256 tokens  16.3 / 14.6 / 14.1 / 16.3 / 20.5   (384 of 64x64)
+//                   384 tokens  22.0 / 19.8 / 19.0 / 16.9 / 20.8   (576 of 64x64)
+//                   768 tokens  37.9 / 32.0 / 28.1 / 26.9 / 23.3   (144 of 256x128)
+//                  1024 tokens  48.6 / 39.3 / 33.1 / 28.0 / 26.5
+//   Q4_K 3584 rows 1024 tokens  32.4 / 27.2 / 24.4 / 19.9 / 23.6   (112 of 256x128)
+//   Q5_K 6144 rows  256 tokens  17.5 / 15.1 / 14.9 / 17.2 / 21.7
+//                   768 tokens  42.5 / 33.6 / 29.9 / 27.7 / 24.4
 // Q6_K decodes at twice the cost per weight, so that its 64x64 tile loses to
 // 64x128 (one decode per four MFMAs) beyond 256 workgroups (2048 rows, 768
-// tokens: 22.3 against 19.9 us), and with many column blocks, where 64x128 tiles
-// are too few, to dequantizing the matrix once (1024 x 3584, 768 tokens: 33.0
-// against 25.5 us; 1024 x 2048, 1024 tokens: 24.4 against 20.9 us).
+// tokens: 22.1 against 19.5 us), and with many column blocks, where 64x128 tiles
+// are too few, to dequantizing the matrix once (1024 x 3584, 768 tokens: 32.4
+// against 25.3 us).
 MmForm mm_form(int format, uint64_t rows, uint64_t cols, uint64_t tokens) {
   auto grid = [&](uint64_t r, uint64_t t) { return (rows + r - 1) / r * ((tokens + t - 1) / t); };
   if (grid(32, 32) <= 256) {
@@ -725,6 +727,45 @@ MmForm mm_form(int format, uint64_t rows, uint64_t cols, uint64_t tokens) {
   return grid(256, 128) > 128 ? MmForm::lds_256 : MmForm::lds_128;
 }
 
+// The estimated time of the two launches in us, for the forms of more than 256 tiles
+// of 32 x 64: packing, the output, and per round of 256 workgroups the K blocks that
+// a wave walks.  Fitted to 3855 products (512 to 24576 rows, 256 to 12288 columns, 65
+// to 2048 tokens): 8% off (rms), kquant_matmul_us 5%.  Where many tokens share the
+// weights, decoding them once per 64 or 128 tokens costs more than dequantizing them
+// first or than the B tile's decode; those forms / these tiles, us:
+//   Q6_K 6144 x 1024, 1024 tokens  28.3 / 31.1     2048 x 1024, 1024  18.8 / 19.8
+//   Q5_K 6144 x 2048, 1024 tokens  43.2 / 44.1     2048 x 6144,  700  49.1 / 53.5
+//   Q4_K 8192 x 256,   512 tokens (B tile)  9.0 / 10.9
+// By this rule 38 of the 3855 take these tiles where they are more than 3% slower, at
+// most 17%; without it 647 did, at most 48%.
+double mm_us(MmForm form, int format, size_t count, const size_t* rows, size_t cols,
+             size_t tokens) {
+  struct Cost {
+    uint64_t rows, tokens;
+    double block[3];  // per K block (per four, split over the waves), by format
+    double round;
+  };
+  const Cost c = form == MmForm::split_64x64 ? Cost{64, 64, {2.7, 3.1, 6.25}, 0.0}
+                 : form == MmForm::lds_64    ? Cost{64, 128, {0.0, 0.0, 2.3}, 1.8}
+                 : form == MmForm::lds_128   ? Cost{128, 128, {1.85, 2.2, 2.9}, 0.65}
+                                             : Cost{256, 128, {3.25, 3.8, 4.95}, 0.5};
+  uint64_t tiles = 0;
+  double outputs = 0.0;
+  for (size_t i = 0; i < count; ++i) {
+    tiles += (rows[i] + c.rows - 1) / c.rows;
+    outputs += 1e-6 * (double)rows[i] * (double)tokens;
+  }
+  const double rounds = (double)((tiles * ((tokens + c.tokens - 1) / c.tokens) + 255) / 256);
+  const uint64_t nb = cols / 256;
+  // Fewer blocks than waves, or than the pipeline of a Q6_K chain needs to fill.
+  double walk = nb == 1 && format == 2 ? 1.3 : (double)nb;
+  if (form == MmForm::split_64x64) {
+    walk = nb < 4 ? (double)(nb + 3) / 7.0 : (double)((nb + 3) / 4);
+  }
+  return 5.0 + 2.6e-6 * (double)tokens * (double)cols + 0.82 * outputs +
+         rounds * (walk * c.block[format] + c.round);
+}
+
 template <int F>
 hipError_t launch_form(MmForm form, const MmArgs& a, hipStream_t stream) {
   switch (form) {
@@ -746,11 +787,19 @@ hipError_t launch_form(MmForm form, const MmArgs& a, hipStream_t stream) {
 
 }  // namespace
 
-bool kquant_mm_supported(int format, size_t rows, size_t cols, size_t tokens) {
+bool kquant_mm_supported(int format, size_t count, const size_t* rows, size_t cols,
+                         size_t tokens) {
   // 32-bit lane offsets within a tile's rows.
-  return tokens > kKquantGemvMaxTokens &&
-         (uint64_t)cols / 256u * kquant_block_bytes(format) * 256u < (1ull << 31) &&
-         mm_form(format, rows, cols, tokens) != MmForm::two_pass;
+  if (tokens <= kKquantGemvMaxTokens ||
+      (uint64_t)cols / 256u * kquant_block_bytes(format) * 256u >= (1ull << 31)) {
+    return false;
+  }
+  const MmForm form = mm_form(format, *std::max_element(rows, rows + count), cols, tokens);
+  if (form == MmForm::split_32x32 || form == MmForm::split_32x64) {
+    return true;
+  }
+  return form != MmForm::two_pass && mm_us(form, format, count, rows, cols, tokens) <=
+                                       0.98 * kquant_matmul_us(format, count, rows, cols, tokens);
 }
 
 size_t kquant_mm_workspace_bytes(size_t cols, size_t tokens) {

@@ -56,6 +56,7 @@ def test_split_tiles_against_two_pass(ops, monkeypatch, fmt, rows, cols, tokens)
     (3585, 1024, 777),   # 128-row tiles, one row and nine tokens past them
     (6100, 512, 900),    # 256-row tiles, partial
     (4100, 256, 640),    # one K block: fewer stages than the pipeline holds
+    (4100, 256, 900),    # the same in 256-row tiles (Q4_K, Q5_K)
 ])
 def test_chain_tiles_equal_two_pass(ops, monkeypatch, fmt, rows, cols, tokens):
     print(f"mm chain {fmt} {rows}x{cols} tokens={tokens}", flush=True)
@@ -67,14 +68,37 @@ def test_chain_tiles_equal_two_pass(ops, monkeypatch, fmt, rows, cols, tokens):
 
 
 @pytest.mark.gpu
-def test_q6_chain_tile_of_64_rows_equals_two_pass(ops, monkeypatch):
-    rows, cols, tokens = 4090, 1280, 500
+@pytest.mark.parametrize("rows,cols,tokens", [
+    (4090, 1280, 500),                      # 64-row tiles
+    (6100, 512, 257), (12290, 256, 130),    # 128
+    (12290, 256, 257), (16390, 512, 200),   # 256
+])
+def test_q6_chain_tiles_equal_two_pass(ops, monkeypatch, rows, cols, tokens):
+    """The shapes for which Q6_K takes them: elsewhere its many-token products stay
+    with the two-pass form (mm_us in kquant_mm.hip)."""
     print(f"mm chain q6_k {rows}x{cols} tokens={tokens}", flush=True)
     w, x = operands("q6_k", rows, cols, tokens)
     got = ops.kquant_matmul("q6_k", w, rows, cols, x, tokens)
     monkeypatch.setenv("KRAKEN_KQUANT_GEMM", "unfused")
     two_pass = ops.kquant_matmul("q6_k", w, rows, cols, x, tokens)
     np.testing.assert_array_equal(got.view(np.uint32), two_pass.view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt,rows,cols,tokens", [
+    ("q4_k", 8192, 256, 512), ("q4_k", 8192, 256, 513),      # B tile; 256-row tiles
+    ("q5_k", 1024, 3584, 512), ("q5_k", 1024, 3584, 513),    # 32 x 64; two passes, K split
+    ("q6_k", 6144, 1024, 567), ("q6_k", 6144, 1024, 568),    # 128 rows; two passes
+])
+def test_either_side_of_the_estimates(ops, monkeypatch, fmt, rows, cols, tokens):
+    """Shapes next to each other that the estimated times send to different forms."""
+    print(f"mm estimates {fmt} {rows}x{cols} tokens={tokens}", flush=True)
+    w, x = operands(fmt, rows, cols, tokens)
+    got = ops.kquant_matmul(fmt, w, rows, cols, x, tokens)
+    monkeypatch.setenv("KRAKEN_KQUANT_GEMM", "unfused")
+    two_pass = ops.kquant_matmul(fmt, w, rows, cols, x, tokens)
+    scale = np.abs(two_pass).mean() * np.sqrt(cols)
+    assert np.abs(got - two_pass).max() <= 2 * TOL * scale
 
 
 @pytest.mark.gpu
