@@ -61,12 +61,16 @@ def test_gdn_state_offset_and_neighbours_untouched(hip_ctx):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tokens,prefill", [(97, None), (97, "chunked"), (200, None)])
 @pytest.mark.parametrize("offset_extra", [0, 1])
-def test_gdn_prefill_state_offset_d128(hip_ctx, offset_extra):
+def test_gdn_prefill_state_offset_d128(hip_ctx, monkeypatch, offset_extra, tokens, prefill):
     """head_dim 128 multi-token calls at a state offset: a 16-byte aligned offset
-    takes the LDS-staged prefill kernel, an odd one the generic kernel; both must
-    update exactly their own state block."""
-    tokens, h, d = 97, 4, 128
+    takes the LDS-staged prefill kernel (97 tokens) or the chunked kernels (forced,
+    and 200 tokens), an odd one the generic kernel; each must update exactly its own
+    state block."""
+    if prefill is not None:
+        monkeypatch.setenv("KRAKEN_GDN_PREFILL", prefill)
+    h, d = 4, 128
     q, k, v, g, b, _ = gdn_inputs(12, tokens, h, h, d)
     blk = h * d * d
     big = (0.1 * np.random.default_rng(13).standard_normal(3 * blk + 4)).astype(np.float32)
@@ -83,17 +87,17 @@ def test_gdn_prefill_state_offset_d128(hip_ctx, offset_extra):
 @pytest.mark.gpu
 @pytest.mark.parametrize("tokens", [64, 257, 1024])
 def test_gdn_prefill_kernels_agree(hip_ctx, monkeypatch, tokens):
-    """The three multi-token kernels for head_dim 128 -- chunked WY (default),
-    LDS-staged sequential (KRAKEN_GDN_PREFILL=sequential) and the generic
-    recurrence (KRAKEN_GDN_PREFILL=generic) -- give the same outputs and state,
-    and each matches the oracle."""
+    """The three multi-token kernels for head_dim 128 -- chunked WY, LDS-staged
+    sequential and the generic recurrence, each forced by KRAKEN_GDN_PREFILL -- and
+    the default (sequential for 64 tokens here, chunked for more) give the same
+    outputs and state, and each matches the oracle."""
     hk = hv = 16
     d = 128
     q, k, v, g, b, s = gdn_inputs(14, tokens, hk, hv, d, state_scale=0.1)
     ops = kh.NumpyOps(hip_ctx)
     out_ref, st_ref = oracle.gated_delta_net(q, k, v, g, b, s, tokens, hk, hv, d)
     results = {}
-    for mode in (None, "sequential", "generic"):
+    for mode in (None, "chunked", "sequential", "generic"):
         if mode is None:
             monkeypatch.delenv("KRAKEN_GDN_PREFILL", raising=False)
         else:
@@ -102,9 +106,11 @@ def test_gdn_prefill_kernels_agree(hip_ctx, monkeypatch, tokens):
         np.testing.assert_allclose(results[mode][0], out_ref, rtol=0, atol=ATOL, err_msg=str(mode))
         np.testing.assert_allclose(results[mode][1], st_ref, rtol=0, atol=ATOL, err_msg=str(mode))
     monkeypatch.delenv("KRAKEN_GDN_PREFILL", raising=False)
-    for mode in ("sequential", "generic"):
-        np.testing.assert_allclose(results[None][0], results[mode][0], rtol=0, atol=2e-5)
-        np.testing.assert_allclose(results[None][1], results[mode][1], rtol=0, atol=2e-5)
+    for mode in (None, "sequential", "generic"):
+        np.testing.assert_allclose(results["chunked"][0], results[mode][0], rtol=0, atol=2e-5)
+        np.testing.assert_allclose(results["chunked"][1], results[mode][1], rtol=0, atol=2e-5)
+    default = "sequential" if tokens == 64 else "chunked"
+    np.testing.assert_array_equal(results[None][0], results[default][0])
 
 
 @pytest.mark.gpu
@@ -243,10 +249,13 @@ def test_unfused_conv_ops_match_oracle(hip_ctx):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tokens", [1, 64, 300])
-def test_gdn_gated_fused_matches_reference_chain(hip_ctx, tokens):
+@pytest.mark.parametrize("tokens,prefill", [(1, None), (64, None), (300, None), (64, "chunked"),
+                                            (101, "chunked")])
+def test_gdn_gated_fused_matches_reference_chain(hip_ctx, monkeypatch, tokens, prefill):
     """prepare_gate_beta + GDN + norm-gated epilogue fused vs the reference op chain
     (qwen35_runtime.cpp:2913-3008) on the oracle."""
+    if prefill is not None:
+        monkeypatch.setenv("KRAKEN_GDN_PREFILL", prefill)
     hk = hv = 16
     d = 128
     rng = np.random.default_rng(7)

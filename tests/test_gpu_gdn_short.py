@@ -30,13 +30,16 @@ def test_short_chunks_against_oracle(hip_ctx, tokens, hk, hv):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tokens", [64, 100, 160])
-def test_chunked_kernels_below_their_rule(hip_ctx, monkeypatch, tokens):
-    print(f"gdn chunked tokens={tokens}", flush=True)
-    args = gdn_inputs(tokens, tokens, 16, 16, 128, state_scale=0.1)
+@pytest.mark.parametrize("tokens,hk,hv", [
+    (64, 16, 16), (100, 16, 16), (160, 16, 16),
+    (64, 2, 4), (130, 2, 6),   # grouped heads, a partial last chunk
+])
+def test_chunked_kernels_below_their_rule(hip_ctx, monkeypatch, tokens, hk, hv):
+    print(f"gdn chunked tokens={tokens} heads={hk}/{hv}", flush=True)
+    args = gdn_inputs(tokens, tokens, hk, hv, 128, state_scale=0.1)
     monkeypatch.setenv("KRAKEN_GDN_PREFILL", "chunked")
-    out, state = kh.NumpyOps(hip_ctx).gated_delta_net(*args, tokens, 16, 16, 128)
-    want, want_state = oracle.gated_delta_net(*args, tokens, 16, 16, 128)
+    out, state = kh.NumpyOps(hip_ctx).gated_delta_net(*args, tokens, hk, hv, 128)
+    want, want_state = oracle.gated_delta_net(*args, tokens, hk, hv, 128)
     np.testing.assert_allclose(out, want, rtol=0, atol=1e-4)
     np.testing.assert_allclose(state, want_state, rtol=0, atol=1e-4)
 

@@ -222,6 +222,15 @@ def test_pipelined_gemm_equals_plain_gemm(ops, monkeypatch, fmt, rows, cols, tok
 GGML = {"q4_k": 12, "q5_k": 13, "q6_k": 14}
 
 
+@pytest.fixture(params=[None, "fused", "unfused"])
+def gemm_form(request, monkeypatch):
+    """The library's own choice between the GEMM forms, and each older form for
+    every format (KRAKEN_KQUANT_GEMM): the choice leaves them only some shapes."""
+    if request.param is not None:
+        monkeypatch.setenv("KRAKEN_KQUANT_GEMM", request.param)
+    return request.param
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("group,tokens", [
     ((("q4_k", 2048), ("q4_k", 16), ("q4_k", 16)), 1024),   # prefill z, beta, alpha
@@ -229,13 +238,15 @@ GGML = {"q4_k": 12, "q5_k": 13, "q6_k": 14}
     ((("q4_k", 3584), ("q4_k", 3584)), 1024),                # FFN up, gate
     ((("q4_k", 130), ("q4_k", 300), ("q4_k", 16), ("q4_k", 1)), 200),  # ragged tiles
     ((("q5_k", 6144), ("q4_k", 2048)), 1024),                # mixed types: one call each
+    ((("q5_k", 512), ("q5_k", 130)), 300),
+    ((("q6_k", 512), ("q6_k", 130)), 300),
 ])
-def test_multi_matmul_equals_single_matmuls(hip_ctx, ops, group, tokens):
+def test_multi_matmul_equals_single_matmuls(hip_ctx, ops, gemm_form, group, tokens):
     """kraken_hip_kquant_matmul_multi_f32 against each matrix's own matmul
-    entry on the same input: bit-identical where the single call runs without a
-    K split (the grouped launch never splits), else within TOL of the oracle
-    like the single call (K split into planes sums in another order)."""
-    print(f"multi matmul {group} tokens={tokens}", flush=True)
+    entry on the same input: bit-identical for a matrix of 128 x 128 tiles enough
+    that neither call splits K, else within TOL of the oracle like the single call
+    (a K split sums in another order)."""
+    print(f"multi matmul {group} tokens={tokens} form={gemm_form}", flush=True)
     cols = 1024
     x = np.random.default_rng(tokens).standard_normal(tokens * cols).astype(np.float32)
     ws = [kc.random_weight_fast(f, r, cols, seed=31 * i + r) for i, (f, r) in enumerate(group)]
@@ -247,7 +258,7 @@ def test_multi_matmul_equals_single_matmuls(hip_ctx, ops, group, tokens):
         got = ob.download(tokens * r)
         single = ops.kquant_matmul(f, w, r, cols, x, tokens)
         tiles = -(-r // 128) * -(-tokens // 128)
-        if f == "q4_k" and tiles < 128 and tokens > 8:
+        if tiles < 128 and tokens > 8:
             want, scale = oracle_projection(f, w, r, cols, x, tokens)
             check_projection(got, want, scale, f"{f} {r} rows")
         else:
@@ -259,13 +270,13 @@ def test_multi_matmul_equals_single_matmuls(hip_ctx, ops, group, tokens):
 @pytest.mark.parametrize("fmt,rows,cols", [("q6_k", 1024, 3584), ("q4_k", 1024, 2048),
                                            ("q4_k", 3584, 1024), ("q5_k", 6144, 1024)])
 @pytest.mark.parametrize("tokens", [9, 1024])
-def test_fused_matmul_equals_separate_ops(hip_ctx, fmt, rows, cols, tokens):
+def test_fused_matmul_equals_separate_ops(hip_ctx, gemm_form, fmt, rows, cols, tokens):
     """kraken_hip_kquant_matmul_fused_f32 against the ops it folds:
     silu_mul_f32_in_place(gate, up), the matmul entry, add_f32_in_place(residual,
     out).  Bit-identical with SwiGLU, with the residual (given as the output
     buffer itself, and as a separate buffer), with both and with neither, with
-    and without K splits, in both GEMM forms."""
-    print(f"fused matmul {fmt} {rows}x{cols} tokens={tokens}", flush=True)
+    and without K splits, in every GEMM form."""
+    print(f"fused matmul {fmt} {rows}x{cols} tokens={tokens} form={gemm_form}", flush=True)
     rng = np.random.default_rng(rows + tokens)
     w = hip_ctx.buffer(kc.random_weight_fast(fmt, rows, cols, seed=rows + cols))
     gate = rng.standard_normal(tokens * cols).astype(np.float32)

@@ -142,7 +142,7 @@ def _read(d, name, dtype):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tokens,layer", [(1, 5), (80, 1), (7, 17)])
+@pytest.mark.parametrize("tokens,layer", [(1, 5), (80, 1), (7, 17), (200, 2)])
 @pytest.mark.parametrize("order", ["reference", "fused"])
 def test_linear_attention_driver_matches_oracle_chain(order, tokens, layer):
     rng = np.random.default_rng(100 + tokens)
