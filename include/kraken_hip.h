@@ -640,7 +640,9 @@ KRAKEN_API int kraken_hip_kquant_matvec_multi_f32(
  * input otherwise; residual may be empty (then 0) or the output buffer itself
  * (add_f32_in_place), but no other view that overlaps the output.  The same
  * bits as the separate ops.  More than 8 tokens (the GEMM path); up and
- * residual 16-byte aligned; a given up takes the two-pass GEMM form. */
+ * residual 16-byte aligned.  Uses context workspace: the fp16 inputs, and for
+ * the forms that dequantize the matrix first or split K over workgroups the
+ * fp16 matrix and the partial planes. */
 KRAKEN_API int kraken_hip_kquant_matmul_fused_f32(kraken_hip_context* context, uint32_t ggml_type,
                                                   kraken_buffer weight, size_t rows, size_t cols,
                                                   size_t tokens, kraken_buffer input,
@@ -652,13 +654,14 @@ KRAKEN_API int kraken_hip_kquant_matmul_fused_f32(kraken_hip_context* context, u
  * and alpha; the FFN up and gate).  Arrays of `count` (1..4) entries give each
  * matrix's GGUF type (12 Q4_K, 13 Q5_K, 14 Q6_K), weight, rows and output
  * [tokens][rows]; each is checked as its matmul entry checks it.  When every
- * matrix has the same type, more than 8 tokens and the type takes the GEMM
- * form that decodes the weights in its B tile (Q4_K by default), the matrices
- * run as one launch with no K split; otherwise, or with
- * KRAKEN_KQUANT_GROUP=off, each runs as its matmul entry.  A matrix whose own
- * entry would split K then sums in another order: within fp32 rounding of its
- * separate result, bit-identical to it when it would not split.  Outputs must
- * not overlap each other or the input. */
+ * matrix has the same type and more than 8 tokens, the matrices share the tiles
+ * that suit the largest of them: one launch rounds the input to fp16 in the
+ * context workspace, one multiplies (any type; Q4_K may run as one launch that
+ * decodes the weights in its B tile instead).  Where that is not the faster
+ * form, or with KRAKEN_KQUANT_GROUP=off, each runs as its matmul entry.  Either
+ * form may sum K in another order than the matrix's own entry: within fp32
+ * rounding of its separate result.  Outputs must not overlap each other or the
+ * input. */
 KRAKEN_API int kraken_hip_kquant_matmul_multi_f32(kraken_hip_context* context, size_t count,
                                                   const uint32_t* ggml_types,
                                                   const kraken_buffer* weights,

@@ -33,9 +33,7 @@ struct DecodeParams {
   // Ragged mode: dense work list, one item per workgroup (blockIdx.x):
   // {token, kv_head << 16 | split}, token 0xffffffff past the last item.
   const uint2* work_items;
-  // A several-token kernel (attention_rows.hip, attention_rows_f32.hip); last, as in
-  // front of scale_log2 it cost the ragged step of 64 sequences 0.4%.
-  bool rows;
+  bool rows;  // a several-token kernel (attention_rows.hip, attention_rows_f32.hip)
 };
 
 // Keys of token t (positions table in ragged mode); at least 1 (a position of

@@ -340,8 +340,9 @@ hipError_t launch_attention_prologue_decode(const PrologueArgs& a, uint32_t laye
 
 // K-quant projections (kquant.hip).  format: 0 = Q4_K, 1 = Q5_K, 2 = Q6_K;
 // weights are row-major blocks (cols / 256 per row).  Up to
-// kKquantGemvMaxTokens tokens take the fp32 GEMV; more take the fp16 MFMA
-// GEMM, which stages fp16 weights and inputs in the workspace.
+// kKquantGemvMaxTokens tokens take the fp32 GEMV; more an fp16 MFMA GEMM:
+// kquant_mm.hip's, or one of the older forms, of which the two-pass one stages
+// fp16 weights and inputs in the workspace.
 constexpr size_t kKquantGemvMaxTokens = 8;
 // Matrices per grouped GEMM launch (launch_kquant_matmul_group).
 constexpr size_t kKquantGroupMax = 4;

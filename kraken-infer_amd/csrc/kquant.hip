@@ -1517,7 +1517,8 @@ __global__ __launch_bounds__(256) void gemm_f16_pipe_kernel(const half_t* x, con
 // then RNE to fp16), so the B tile holds the values the unfused pass wrote,
 // and the MFMAs run over K in the same order: the result equals the unfused
 // path's.  Rows past the matrix decode its last row (never stored).  16-byte
-// chunk j of an LDS row lives at j ^ (row & 15).
+// chunk j of an LDS row lives at j ^ (row & 15).  Q5_K and Q6_K run it only with
+// KRAKEN_KQUANT_GEMM=fused.
 constexpr int kQK = 128;
 
 // Several matrices of one format that multiply the same input, in one grid:
@@ -2098,7 +2099,8 @@ uint32_t kquant_block_bytes(int format) {
   return format == 0 ? 144u : (format == 1 ? 176u : (format == 2 ? 210u : 0u));
 }
 
-// The GEMM form per format: the fused one (weights decoded in the B tile) for
+// The form of launch_kquant_matmul per format (whether it or kquant_mm.hip's two
+// launches run: kquant_mm_supported): the fused one (weights decoded in the B tile) for
 // Q4_K, the two-pass one (the weights dequantized to an fp16 matrix in the
 // workspace, then the fp16 GEMM) for Q5_K and Q6_K, whose decode costs more
 // VALU work per weight than the fused tile hides under its MFMAs (measured on
