@@ -124,7 +124,7 @@ struct RowsPlace {
   uint32_t unit, order;
 };
 __host__ __device__ __forceinline__ bool rows_by_xcd(uint32_t units, uint32_t groups) {
-  return units % 8u == 0u && groups < 65536u;  // groups: a grid's y
+  return units % 8u == 0u && groups < 65536u && units < 8u * 65536u;  // a grid's y and z
 }
 __device__ __forceinline__ RowsPlace place_rows(uint32_t units, uint32_t groups) {
   if (rows_by_xcd(units, groups)) {
